@@ -277,20 +277,18 @@ DR_INLINE float node_importance_len(const DrEdgeNode &n, float bound, F3 p, floa
 // walk; a selected edge's ordinal is its index in the tree with bit 30 set
 // for the "all" pass: the tree is stored in depth-first order (left child
 // first, leaves' edges in leaf order), so ordinals sort like the reference's
-// sequential order of selection.  The traversal is explicit state advanced
-// one node per et_step() so that a persistent kernel can give a lane a new
-// point as soon as its traversal ends; et_step() calls
-// `emit(weight, in_normal_tree, index, ordinal)` per selected edge.
+// sequential order of selection.  et_expand() expands one node,
+// et_leaf_edge() calls `emit(weight, in_normal_tree, index, ordinal)` per
+// selected edge of a leaf.
 //
-// The stack is an object of its own (owned by the caller), not a member of
-// EdgeTraversal: its storage is indexed at run time, while every other field
-// of the traversal state stays in registers.  An entry carries what the parent
-// already knew of the node (child offset, edge count, what its bound and
-// whether the point lies in its box decide), so popping an interior node needs
-// only its two children's records, loaded side by side.  Two stacks:
-// LdsStack (the selection kernel): the top entries live in LDS and older ones
-// spill to private memory in halves; and PlainStack, an array, against which
-// the stack self-test (k_tree_stack) checks it.
+// Nodes of one point's walk are independent of each other (keyed draws), so
+// who expands them, and when, does not matter.  The selection kernel keeps the
+// pending nodes of all of a wave's points in one stack (WaveStack) from which
+// idle lanes take their next node; the breadth-first kernels keep one list per
+// tree level.  An entry carries what the parent already knew of the node (child
+// offset, edge count, what its bound and whether the point lies in its box
+// decide), so expanding it needs only its two children's records, loaded side
+// by side.
 //
 // An entry is 16 bytes.  What popping needs of the node's bound is two flags,
 // kept in the sign bits of the two pmfs (a pmf is never negative):
@@ -319,74 +317,81 @@ struct TreeAlt {
     float cone, all;
 };
 
-struct PlainStack {
-    TreeEntry e[DR_TREE_STACK];
-    TreeAlt alt[DR_TREE_STACK];
-    int sp;
-    DR_INLINE void clear() { sp = 0; }
-    DR_INLINE int size() const { return sp; }
-    DR_INLINE void push(const TreeEntry &x, TreeAlt a, bool with_alt) {
-        if (with_alt) alt[sp] = a;
-        e[sp++] = x;
+// A stack of WORDS-word entries shared by the 64 lanes of a wave.  The top of
+// it, at most DR_WSTACK_LDS entries, lives in LDS (a ring, one row per word:
+// neighbouring entries lie in neighbouring banks); when a push would overflow
+// the ring its bottom 64 entries move to private memory, one entry per lane
+// (coalesced), and come back as a block once the ring holds too few for a
+// pop.  Every lane of the wave calls push and pop together.  When all blocks
+// nearly in use, throttled() asks the caller to let lane 0 alone pop, expand
+// and push: a depth-first walk adds at most one entry per tree level, for which
+// there is room beside one push of all lanes.
+#define DR_WSTACK_LDS 128
+#define DR_WSTACK_BLOCKS 30
+#define DR_WSTACK_CAP (DR_WSTACK_BLOCKS * 64 + DR_WSTACK_LDS)  // 32 entries per lane
+static_assert(DR_TREE_STACK <= 32, "throttled() leaves room for 32 entries of one lane's walk");
+DR_INLINE void wave_lds_fence() {
+#if defined(__HIP_DEVICE_COMPILE__)
+    // orders the wave's LDS accesses for the compiler (the hardware runs a
+    // wave's LDS instructions in order)
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+#endif
+}
+template <int WORDS>
+struct WaveStack {
+    DR_LDS uint32_t *w;  // [WORDS][DR_WSTACK_LDS]
+    int n, base;         // entries in LDS: ring positions base .. base + n - 1
+    int blocks;          // blocks of 64 entries in `spill`
+    uint32_t spill[DR_WSTACK_BLOCKS * WORDS];
+    DR_INLINE void init(DR_LDS uint32_t *lds) {
+        w = lds;
+        n = base = blocks = 0;
     }
-    DR_INLINE TreeEntry pop(TreeAlt &a, bool with_alt) {
-        --sp;
-        if (with_alt) a = alt[sp];
-        return e[sp];
-    }
-};
-
-// entries per lane in LDS: 10 x 16 B x 256 lanes = 40 KB per workgroup, so
-// that four workgroups (4 waves per SIMD) share a CU's 160 KB; 12 entries
-// (48 KB, 3 waves per SIMD) made k_select 8 % slower
-#define DR_LDS_STACK 10
-#define DR_LDS_WORDS 4   // words per entry
-
-// Top DR_LDS_STACK entries of each lane in LDS, one word of an entry per
-// row of the block's lanes (conflict-free: lane l always uses bank l % 64);
-// entries below them in private memory.  Entries [lo, sp) are in LDS, entry i
-// in slot i % DR_LDS_STACK; [0, lo) in `spill`.  A push onto a full LDS part
-// moves its bottom entry to `spill`; a pop below lo takes the entry from
-// `spill` directly, so an entry goes to private memory at most once and
-// comes back at most once (the walk is depth first: once entries below the
-// LDS part are being popped, everything above them has been).
-struct LdsStack {
-    DR_LDS float *lds;  // the block's stack area + threadIdx.x (stride: blockDim.x)
-    int stride;
-    TreeEntry spill[DR_TREE_STACK];
-    TreeAlt alt[DR_TREE_STACK];
-    int sp, lo;
-    DR_INLINE void clear() { sp = lo = 0; }
-    DR_INLINE int size() const { return sp; }
-    DR_INLINE void put(int slot, const TreeEntry &x) {
-        DR_LDS float *w = lds + slot * DR_LDS_WORDS * stride;
-        w[0] = __int_as_float(x.code);
-        w[stride] = __uint_as_float(x.cpmf);
-        w[2 * stride] = __uint_as_float(x.apmf);
-        w[3 * stride] = __int_as_float(x.off);
-    }
-    DR_INLINE TreeEntry get(int slot) const {
-        const DR_LDS float *w = lds + slot * DR_LDS_WORDS * stride;
-        return TreeEntry{__float_as_int(w[0]), __float_as_uint(w[stride]), __float_as_uint(w[2 * stride]),
-                         __float_as_int(w[3 * stride])};
-    }
-    DR_INLINE void push(const TreeEntry &x, TreeAlt a, bool with_alt) {
-        if (sp - lo == DR_LDS_STACK) {
-            spill[lo] = get(lo % DR_LDS_STACK);
-            lo++;
+    DR_INLINE int size() const { return n + 64 * blocks; }
+    DR_INLINE bool throttled() const { return size() > DR_WSTACK_CAP - 64 - 32; }
+    // lanes with `have` push their entry, lower lanes below higher ones
+    DR_INLINE void push(bool have, const uint32_t *x, int lane) {
+        unsigned long long m = __ballot(have);
+        int k = __popcll(m);
+        if (k == 0) return;
+        if (n + k > DR_WSTACK_LDS) {
+            int i = (base + lane) & (DR_WSTACK_LDS - 1);
+            for (int r = 0; r < WORDS; r++) spill[blocks * WORDS + r] = w[r * DR_WSTACK_LDS + i];
+            blocks++;
+            base = (base + 64) & (DR_WSTACK_LDS - 1);
+            n -= 64;
+            wave_lds_fence();
         }
-        if (with_alt) alt[sp] = a;
-        put(sp % DR_LDS_STACK, x);
-        sp++;
-    }
-    DR_INLINE TreeEntry pop(TreeAlt &a, bool with_alt) {
-        --sp;
-        if (with_alt) a = alt[sp];
-        if (sp < lo) {
-            lo = sp;
-            return spill[sp];
+        if (have) {
+            int i = (base + n + __popcll(m & ((1ull << lane) - 1ull))) & (DR_WSTACK_LDS - 1);
+            for (int r = 0; r < WORDS; r++) w[r * DR_WSTACK_LDS + i] = x[r];
         }
-        return get(sp % DR_LDS_STACK);
+        n += k;
+        wave_lds_fence();
+    }
+    // lanes with `want` take entries from the top, lower lanes first; true
+    // for the lanes that got one
+    DR_INLINE bool pop(bool want, uint32_t *x, int lane) {
+        unsigned long long m = __ballot(want);
+        int k = __popcll(m);
+        if (n < k && blocks > 0) {
+            blocks--;
+            base = (base - 64) & (DR_WSTACK_LDS - 1);
+            int i = (base + lane) & (DR_WSTACK_LDS - 1);
+            for (int r = 0; r < WORDS; r++) w[r * DR_WSTACK_LDS + i] = spill[blocks * WORDS + r];
+            n += 64;
+            wave_lds_fence();
+        }
+        int rank = __popcll(m & ((1ull << lane) - 1ull));
+        bool got = want && rank < n;
+        if (got) {
+            int i = (base + n - 1 - rank) & (DR_WSTACK_LDS - 1);
+            for (int r = 0; r < WORDS; r++) x[r] = w[r * DR_WSTACK_LDS + i];
+        }
+        n -= min(k, n);
+        wave_lds_fence();
+        return got;
     }
 };
 
@@ -403,8 +408,6 @@ struct EdgeTraversal {
     // learned mixture, 1 = this point uses the learned node lengths, 2 = the
     // plain ones (probabilities 0.8 / 0.2)
     int mode;
-    int pops;
-    uint32_t n_inner, n_edges;
     bool cone_pmf_quirk;  // DR_QUIRK_CONE_PMF
 };
 
@@ -468,9 +471,6 @@ DR_INLINE bool et_init(EdgeTraversal &T, Stack &stack, const DrSceneView &S, F3 
     T.cone = cone;
     const DrEdgeNode &root = T.nodes[0];
     float root_bound = bsdf_bound(root, sp, T.B);
-    T.n_inner = 0;
-    T.n_edges = 0;
-    T.pops = 0;
     T.mode = mode;
     stack.clear();
     stack.push(tree_entry(0, 3, root, root_bound, pmf, pmf, sp.pos), TreeAlt{pmf_o, pmf_o}, mode != 0);
@@ -509,15 +509,6 @@ DR_INLINE void et_leaf_edge(const EdgeTraversal &T, const TreeEntry &e, TreeAlt 
     if (mask & 2) emit(scale * all_pmf / den, T.directional, e.off + i, DR_ORD_ALL_PASS | (e.off + i));
 }
 
-// A leaf's edges in order.
-template <class Emit>
-DR_INLINE void et_leaf(EdgeTraversal &T, const TreeEntry &e, TreeAlt ea, const DrSceneView &S, const SPoint &sp,
-                       Emit &emit) {
-    const int nprims = e.nprims();
-    T.n_edges += nprims;
-    for (int i = 0; i < nprims; i++) et_leaf_edge(T, e, ea, S, sp, i, emit);
-}
-
 // An interior node: the children the passes go on to, at most two, in the
 // order a depth-first walk pushes them (right, then left).  Returns how
 // many (c0 first, then c1).
@@ -527,7 +518,6 @@ DR_INLINE int et_expand(EdgeTraversal &T, const TreeEntry &e, TreeAlt ea, const 
     const float cone_pmf = e.cone_pmf(), all_pmf = e.all_pmf();
     int li = ni + 1, ri = e.off;
     const DrEdgeNode L = gptr(T.nodes)[li], R = gptr(T.nodes)[ri];
-    T.n_inner++;
     bool all_split = e.split_all();
     bool lcs = true, rcs = true;
     if (T.directional) {
@@ -637,41 +627,6 @@ DR_INLINE int et_expand(EdgeTraversal &T, const TreeEntry &e, TreeAlt ea, const 
         n++;
     }
     return n;
-}
-
-// One node.  Returns false when the traversal is done.
-template <class Stack, class Emit>
-DR_INLINE bool et_step(EdgeTraversal &T, Stack &stack, const DrSceneView &S, const SPoint &sp, Emit &emit) {
-    // every node is pushed at most once; the cap guards a malformed tree
-    if (stack.size() == 0 || T.pops >= T.num_nodes + 8) {
-        if (S.stats) {
-            atomicAdd(&S.stats[5], (unsigned long long)T.n_inner);
-            atomicAdd(&S.stats[6], (unsigned long long)T.n_edges);
-        }
-        return false;
-    }
-    T.pops++;
-    TreeAlt ea{0.f, 0.f};
-    TreeEntry e = stack.pop(ea, T.mode != 0);
-    if (e.empty()) return true;
-    if (e.nprims() > 0) {
-        et_leaf(T, e, ea, S, sp, emit);
-        return true;
-    }
-    TreeEntry c0, c1;
-    TreeAlt a0{0.f, 0.f}, a1{0.f, 0.f};
-    int n = et_expand(T, e, ea, S, sp, c0, a0, c1, a1);
-    // the builder bounds the tree depth so that the stack cannot fill (a
-    // full stack would be counted in the statistics, not silently dropped)
-    if (n > 0) {
-        if (stack.size() < DR_TREE_STACK) stack.push(c0, a0, T.mode != 0);
-        else if (S.stats) atomicAdd(&S.stats[7], 1ull);
-    }
-    if (n > 1) {
-        if (stack.size() < DR_TREE_STACK) stack.push(c1, a1, T.mode != 0);
-        else if (S.stats) atomicAdd(&S.stats[7], 1ull);
-    }
-    return true;
 }
 
 struct EdgeResult {

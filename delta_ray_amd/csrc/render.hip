@@ -166,120 +166,7 @@ __global__ void __launch_bounds__(DR_BLOCK) k_path(const DrJob *__restrict__ job
     gc_flush(gkey, gval, DR_GC_SLOTS_BIG, [&](int j) { return jobs[j].grads; });
 }
 
-// B: edge selection, persistent.  Per-point traversal lengths vary by two
-// orders of magnitude (a point inside many node boxes splits at every level),
-// so a lane that has finished its point takes the next one, and every
-// iteration advances each busy lane's traversal by one node.  Starting a point
-// (decoding its slot, the light cone, the material, the root bound) is a long
-// stretch of code that the whole wave executes whenever any lane does, so
-// idle lanes wait until at least `refill` of them are idle (or no lane is
-// busy) and then start new points together.  In a refill, idle lanes take
-// batches of point slots from `work` with one atomic per batch until each has
-// a valid point or the slots run out, so empty slots cost no iteration.
-// Selected edges are appended to the queue in groups of up to DR_EMIT_GROUP
-// per lane (one queue atomic per group; a point's edges flush together at its
-// end, so they sit side by side in the queue, which keeps k_edge's waves on
-// rays from one point: 32 rather than 8 makes k_edge 6 % faster).  Every
-// lane leaves the loop once `work` passes nslots.  cnt[0]: queue length (may
-// exceed cap: the host grows the queue and renders again), cnt[1]: work
-// counter.
-#define DR_EMIT_GROUP 32
-// Points are fetched in the order f in [f_begin, f_end) (a pass's points are
-// f in [0, nslots); a part of them when a pass's selection runs in parts).
-// Four waves per SIMD: the register budget of 128 VGPRs fits the kernel
-// without spills and matches what its LDS stack leaves room for; five (96
-// VGPRs) spill and are 40 % slower.
-__global__ void __launch_bounds__(DR_BLOCK) __attribute__((amdgpu_waves_per_eu(4)))
-k_select(const DrJob *__restrict__ jobs, long long nslots, int maxb, const PointRec *pts, EdgeEntry *q,
-         unsigned long long *cnt, long long cap, int *counts, int refill, long long f_begin, long long f_end) {
-    const long long per_bounce = nslots / maxb;  // nslots is a multiple of maxb
-    __shared__ float s_stack[DR_LDS_STACK * DR_LDS_WORDS * DR_BLOCK];
-    const int lane = (int)__lane_id();
-    EdgeTraversal T;
-    LdsStack stack;
-    stack.lds = (DR_LDS float *)s_stack + threadIdx.x;
-    stack.stride = DR_BLOCK;
-    stack.clear();
-    SPoint sp;
-    const DrSceneView *Sp = &jobs[0].S;
-    long long slot = -1;
-    int j = 0;
-    bool more = true;
-    EdgeEntry buf[DR_EMIT_GROUP];
-    int nbuf = 0;
-    auto flush = [&]() {
-        unsigned long long base = atomicAdd(&cnt[0], (unsigned long long)nbuf);
-        for (int e = 0; e < nbuf; e++)
-            if ((long long)(base + e) < cap) q[base + e] = buf[e];
-        nbuf = 0;
-    };
-    auto emit = [&](float w, bool nrm, int idx, int ord) {
-        // zero-weight edges carry no work (reference delta_ray.cpp:906-908)
-        if (w != 0.f) {
-            buf[nbuf++] = EdgeEntry{(int)slot, idx | (nrm ? (int)0x80000000 : 0), w, ord};
-            if (nbuf == DR_EMIT_GROUP) flush();
-        }
-        j++;
-    };
-    while (true) {
-        unsigned long long idle = __ballot(slot < 0 && more);
-        if (idle && (__popcll(idle) >= refill || __ballot(slot >= 0) == 0)) {
-            // fetch: until every idle lane holds a valid point or the slots run out
-            bool want = slot < 0 && more;
-            long long cand = -1;
-            while (true) {
-                unsigned long long m = __ballot(want);
-                if (!m) break;
-                int leader = __ffsll((long long)m) - 1;
-                unsigned long long base = 0;
-                if (lane == leader) base = atomicAdd(&cnt[1], (unsigned long long)__popcll(m));
-                base = __shfl(base, leader);
-                if (want) {
-                    unsigned long long below = lane == 0 ? 0ull : (m & (~0ull >> (64 - lane)));
-                    long long f = f_begin + (long long)(base + __popcll(below));
-                    // points in the order bounce-major: a wave's points are the
-                    // same bounce of neighbouring samples and pixels, which
-                    // walk similar tree paths (slots are bounce-minor)
-                    long long s = f < f_end ? (f % per_bounce) * maxb + f / per_bounce : nslots;
-                    if (s >= nslots) {
-                        more = false;
-                        want = false;
-                    } else if (pts[s].valid) {  // (only jobs with secondary edges mark points valid)
-                        cand = s;
-                        want = false;
-                    } else {
-                        counts[s] = 0;
-                    }
-                }
-            }
-            // start the new points together
-            if (cand >= 0) {
-                const PointRec &p = pts[cand];
-                const DrJob &J = jobs[p.job];
-                Sp = &J.S;
-                if (select_begin(*Sp, J.c, p, T, stack)) {
-                    slot = cand;
-                    sp = p.sp;
-                    j = 0;
-                } else {
-                    counts[cand] = 0;
-                }
-            }
-        }
-        if (slot < 0) {
-            if (!more) break;
-            continue;
-        }
-        if (!et_step(T, stack, *Sp, sp, emit)) {
-            if (nbuf > 0) flush();
-            counts[slot] = j;
-            if (Sp->stats) atomicAdd(&Sp->stats[3], (unsigned long long)j);
-            slot = -1;
-        }
-    }
-}
-
-// B, breadth first: the same traversal (et_expand / et_leaf, the same keyed
+// B, breadth first: the same traversal (et_expand / et_leaf_edge, the same keyed
 // draws and ordinals, so the same selected edges with the same weights) run
 // one tree level per launch over every point of the pass.  A lane takes one
 // frontier entry (a node some point's passes reached) and expands it, so all
@@ -330,9 +217,6 @@ DR_INLINE void sel_ctx(const SelPoint &P, const DrJob &J, EdgeTraversal &T, SPoi
     T.cone = Cone{P.pos, P.cdir, P.ccos};
     T.mode = (P.info >> 1) & 3;
     T.cone_pmf_quirk = (P.info & 8) != 0;
-    T.pops = 0;
-    T.n_inner = 0;
-    T.n_edges = 0;
     uint64_t sid = (uint64_t)P.sid_lo | ((uint64_t)P.sid_hi << 32);
     philox_init(T.rt, J.c.seed, 0, sid, dr_stream_point_tree((P.info >> 8) & 0xff));
     sp.pos = P.pos;
@@ -540,6 +424,381 @@ __global__ void __launch_bounds__(DR_BLOCK) k_sel_leaves(const DrJob *__restrict
             }
         }
         if (nprims > 0 && J->S.stats) atomicAdd(&J->S.stats[6], (unsigned long long)nprims);
+    }
+}
+
+// The points of a pass (or of the part f in [f_begin, f_end) of it) as a list
+// of their slots, bounce-major: neighbours in the list are the same bounce of
+// neighbouring samples and pixels, which walk similar tree paths (slots are
+// bounce-minor, and those of bounces after a diffuse one are empty: half of the
+// slots at two bounces).  A workgroup lists 2048 slots with one atomic.  Also
+// clears the slots' edge counts.
+#define DR_CNT_POINTS 6                        // word of the counters: points listed
+#define DR_CNT_WORK 16                         // first of the list's eight work counters, 16 words apart
+#define DR_CNT_WORDS (DR_CNT_WORK + 8 * 16)
+#define DR_LIST_PER_THREAD 8
+__global__ void __launch_bounds__(DR_BLOCK) k_sel_points(long long nslots, int maxb, const PointRec *pts, int *list,
+                                                         unsigned long long *cnt, int *counts, long long f_begin,
+                                                         long long f_end) {
+    __shared__ int s_n[DR_LIST_PER_THREAD * (DR_BLOCK / 64)];
+    __shared__ unsigned long long s_base;
+    const long long per_bounce = nslots / maxb;  // nslots is a multiple of maxb
+    const int lane = (int)__lane_id(), w = threadIdx.x >> 6;
+    const long long f0 = f_begin + (long long)blockIdx.x * (DR_BLOCK * DR_LIST_PER_THREAD) + threadIdx.x;
+    int slot[DR_LIST_PER_THREAD], rank[DR_LIST_PER_THREAD];
+    for (int i = 0; i < DR_LIST_PER_THREAD; i++) {
+        long long f = f0 + i * DR_BLOCK;
+        slot[i] = -1;
+        if (f < f_end) {
+            long long s = (f % per_bounce) * maxb + f / per_bounce;
+            counts[s] = 0;
+            if (pts[s].valid) slot[i] = (int)s;  // (only jobs with secondary edges mark points valid)
+        }
+        unsigned long long m = __ballot(slot[i] >= 0);
+        rank[i] = __popcll(m & ((1ull << lane) - 1ull));
+        if (lane == 0) s_n[i * (DR_BLOCK / 64) + w] = __popcll(m);
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        int n = 0;
+        for (int i = 0; i < DR_LIST_PER_THREAD * (DR_BLOCK / 64); i++) {
+            int k = s_n[i];
+            s_n[i] = n;
+            n += k;
+        }
+        s_base = n > 0 ? atomicAdd(&cnt[DR_CNT_POINTS], (unsigned long long)n) : 0ull;
+    }
+    __syncthreads();
+    for (int i = 0; i < DR_LIST_PER_THREAD; i++)
+        if (slot[i] >= 0) list[s_base + s_n[i * (DR_BLOCK / 64) + w] + rank[i]] = slot[i];
+}
+
+// B, depth first: edge selection, persistent, one wave per workgroup.  The
+// length of a point's walk varies by two orders of magnitude and more (a point
+// inside many node boxes splits at every level), so a lane per point leaves
+// most of a wave waiting for its longest walk (27 of 64 lanes active), and a
+// small render waits for single lanes that walk alone.  Here the pending nodes
+// of up to 64 points sit in one stack per wave (WaveStack): every iteration
+// each lane expands one node, whichever point it belongs to, keeps one of its
+// interior children as its next node, and idle lanes take theirs from the
+// stack.  A node's draws are keyed by point and node, so the selected edges do
+// not depend on the order.
+//   * Points: what expanding and testing need of a point (SEL_WORDS words, from
+//     its PointRec and bound_ctx) lies in LDS, a column per point.  A wave
+//     holds two halves of 32 points; a half whose nodes are all done takes new
+//     points while the other half's walk goes on, and points are added whenever
+//     lanes would stay idle, so lanes run dry only at the end of the launch.  The points of a wave belong to one job at a time
+//     (scene pointers and random key stay in scalar registers).
+//   * Leaves wait in a list in LDS until there are 64 of them, so the
+//     silhouette test runs on full waves and a wave's selected edges are
+//     appended to the queue with one atomic.
+// cnt[0]: queue length (may exceed cap: the host grows the queue and selects
+// again), cnt[DR_CNT_POINTS]: points of the list k_sel_points made.  The list is
+// worked off in eight pieces of interleaved blocks, one piece per XCD
+// (workgroups go to the XCDs in turn), each with its own counter in its own
+// cache line, so that fetches do not queue up at one address; a wave whose
+// piece is used up goes on to the next one.  A fetch takes a fortieth of an even share
+// of what is left of the piece, between fetch_min and 64 points: neighbouring
+// points are heavy together (some 20 times the mean walk), and a wave that
+// took many of them last would finish long after the others (with 64 points
+// at any time the waves of the 512 x 512 heightfield ran 59 % of the launch).
+#define SEL_WORDS 28
+template <bool LEARNED>
+__global__ void __launch_bounds__(64)
+k_select(const DrJob *__restrict__ jobs, const int *list, const PointRec *pts, EdgeEntry *q, unsigned long long *cnt,
+         long long cap, int *counts, int fetch_min, int fetch_max) {
+    constexpr int SW = LEARNED ? 7 : 5, LW = LEARNED ? 6 : 4;
+    constexpr int LEAVES = 128;  // 63 waiting and the 64 a round adds
+    __shared__ uint32_t s_point[SEL_WORDS * 64];
+    __shared__ uint32_t s_stack[SW * DR_WSTACK_LDS];
+    __shared__ uint32_t s_leaf[LW * LEAVES];
+    DR_LDS uint32_t *C = (DR_LDS uint32_t *)s_point, *LF = (DR_LDS uint32_t *)s_leaf;
+    const long long npoints = (long long)cnt[DR_CNT_POINTS];
+    const int lane = (int)__lane_id();
+    WaveStack<SW> st;
+    st.init((DR_LDS uint32_t *)s_stack);
+    int nleaf = 0, leaf0 = 0;  // leaves waiting (a ring), the oldest
+    int out0 = 0, out1 = 0; // nodes and leaves pending of either half's points
+    int open = 0, used = 0; // the half that takes new points, its columns taken
+    int job = 0;            // the job of the pending nodes
+    bool more = true;       // points are left to fetch
+    int piece = (int)(blockIdx.x & 7), tried = 0;  // piece of the list, pieces found used up
+    long long left = npoints / 8;                  // points of the piece left at this wave's last fetch
+    const float share = 8.f / (40.f * (float)gridDim.x);
+    long long pending = -1; // a fetched point not started yet
+    bool has = false;       // this lane holds a node
+    uint32_t cur[SW] = {};  // TreeEntry, point [, TreeAlt]
+
+    auto half_count = [&](bool v, uint32_t pt, int &o0, int &o1) {
+        int a = __popcll(__ballot(v)), b = __popcll(__ballot(v && pt >= 32));
+        o0 += a - b;
+        o1 += b;
+    };
+    // a point's constants from its column
+    auto load_point = [&](uint32_t pt, const DrJob &J, EdgeTraversal &T, SPoint &sp) {
+        auto c = [&](int k) { return __uint_as_float(C[k * 64 + pt]); };
+        sp.pos = F3{c(0), c(1), c(2)};
+        F3 n = F3{c(3), c(4), c(5)};
+        sp.ng = n;
+        sp.fr = Frame{F3{0.f, 0.f, 0.f}, F3{0.f, 0.f, 0.f}, n};
+        sp.uv = F2{0.f, 0.f};
+        T.B.hf = Frame{F3{c(6), c(7), c(8)}, F3{c(9), c(10), c(11)}, F3{c(12), c(13), c(14)}};
+        T.B.lx = c(15);
+        T.B.lz = c(16);
+        T.B.lx2 = T.B.lx * T.B.lx;
+        T.B.lz2 = T.B.lz * T.B.lz;
+        T.B.e = c(17);
+        T.B.e2 = T.B.e + 2.f;
+        T.B.dterm = c(18);
+        T.B.slum = c(19);
+        T.cone = Cone{sp.pos, F3{c(20), c(21), c(22)}, c(23)};
+        uint32_t info = C[26 * 64 + pt];
+        bool nrm = (info & 1) != 0;
+        T.nodes = nrm ? J.S.nrm_nodes : J.S.sil_nodes;
+        T.edges = nullptr;
+        T.num_nodes = nrm ? J.S.num_nrm_nodes : J.S.num_sil_nodes;
+        T.directional = nrm;
+        T.mode = LEARNED ? (int)(info >> 1) & 3 : 0;
+        T.cone_pmf_quirk = (J.c.flags & DR_QUIRK_CONE_PMF) != 0;
+        uint64_t sid = (uint64_t)C[24 * 64 + pt] | ((uint64_t)C[25 * 64 + pt] << 32);
+        philox_init(T.rt, J.c.seed, 0, sid, dr_stream_point_tree((int)(info >> 8) & 0xff));
+    };
+    // the oldest `k` (<= 64) waiting leaves: their edges in turn, as many
+    // rounds as the largest of them has edges
+    auto leaves = [&](int k) {
+        wave_lds_fence();
+        const DrJob &J = jobs[job];
+        bool v = lane < k;
+        int i = (leaf0 + lane) & (LEAVES - 1);
+        uint32_t pt = 0, info = 0;
+        TreeEntry te{0, 0u, 0u, 0};
+        TreeAlt ta{0.f, 0.f};
+        int nprims = 0, slot = 0;
+        EdgeTraversal T;
+        SPoint sp;
+        T.directional = false;
+        T.mode = 0;
+        if (v) {
+            // the point's number: 5 bits above the edge index (below 2^27), one in the pmf's sign
+            uint32_t a = LF[2 * LEAVES + i], o = LF[3 * LEAVES + i];
+            te = TreeEntry{(int)LF[i], LF[LEAVES + i], a & 0x7fffffffu, (int)(o & 0x7ffffffu)};
+            pt = (o >> 27) | (a >> 31) << 5;
+            if (LEARNED) ta = TreeAlt{__uint_as_float(LF[(LW - 2) * LEAVES + i]), __uint_as_float(LF[(LW - 1) * LEAVES + i])};
+            nprims = te.nprims();
+            sp.pos = F3{__uint_as_float(C[pt]), __uint_as_float(C[64 + pt]), __uint_as_float(C[128 + pt])};
+            info = C[26 * 64 + pt];
+            slot = (int)C[27 * 64 + pt];
+            T.directional = (info & 1) != 0;
+            if (LEARNED) T.mode = (int)(info >> 1) & 3;
+        }
+        int calls = 0;
+        for (int r = 0; __ballot(r < nprims); r++) {
+            EdgeEntry y0{}, y1{};
+            int ke = 0;
+            if (r < nprims) {
+                auto emit = [&](float w, bool nrm, int idx, int ord) {
+                    calls++;
+                    // zero-weight edges carry no work (reference delta_ray.cpp:906-908)
+                    if (w != 0.f) {
+                        EdgeEntry y{slot, idx | (nrm ? (int)0x80000000 : 0), w, ord};
+                        if (ke == 0) y0 = y;
+                        else y1 = y;
+                        ke++;
+                    }
+                };
+                et_leaf_edge(T, te, ta, J.S, sp, r, emit);
+            }
+            unsigned long long m1 = __ballot(ke >= 1), m2 = __ballot(ke >= 2);
+            int total = __popcll(m1) + __popcll(m2);
+            if (total > 0) {
+                unsigned long long lt = (1ull << lane) - 1ull;
+                unsigned long long b = 0;
+                if (lane == 0) b = atomicAdd(&cnt[0], (unsigned long long)total);
+                long long e = (long long)__shfl(b, 0) + __popcll(m1 & lt) + __popcll(m2 & lt);
+                if (ke > 0 && e < cap) q[e] = y0;
+                if (ke > 1 && e + 1 < cap) q[e + 1] = y1;
+            }
+        }
+        if (J.dx && calls > 0) atomicAdd(&counts[slot], calls);
+        if (J.S.stats) {
+            if (calls > 0) atomicAdd(&J.S.stats[3], (unsigned long long)calls);
+            if (nprims > 0) atomicAdd(&J.S.stats[6], (unsigned long long)nprims);
+        }
+        nleaf -= k;
+        leaf0 = (leaf0 + k) & (LEAVES - 1);
+        int d0 = 0, d1 = 0;
+        half_count(v, pt, d0, d1);
+        out0 -= d0;
+        out1 -= d1;
+    };
+    // lanes with `v` add a leaf to the list
+    auto add_leaf = [&](bool v, const TreeEntry &e, TreeAlt a, uint32_t pt) {
+        unsigned long long m = __ballot(v);
+        if (!m) return;
+        if (v) {
+            int i = (leaf0 + nleaf + __popcll(m & ((1ull << lane) - 1ull))) & (LEAVES - 1);
+            LF[i] = (uint32_t)e.code;
+            LF[LEAVES + i] = e.cpmf;
+            LF[2 * LEAVES + i] = e.apmf | (pt >> 5) << 31;
+            LF[3 * LEAVES + i] = (uint32_t)e.off | pt << 27;
+            if (LEARNED) {
+                LF[(LW - 2) * LEAVES + i] = __float_as_uint(a.cone);
+                LF[(LW - 1) * LEAVES + i] = __float_as_uint(a.all);
+            }
+        }
+        nleaf += __popcll(m);
+        if (nleaf >= 64) leaves(64);
+    };
+    auto pack = [&](uint32_t *x, const TreeEntry &e, TreeAlt a, uint32_t pt) {
+        x[0] = (uint32_t)e.code;
+        x[1] = e.cpmf;
+        x[2] = e.apmf;
+        x[3] = (uint32_t)e.off;
+        x[4] = pt;
+        if (LEARNED) {
+            x[SW - 2] = __float_as_uint(a.cone);
+            x[SW - 1] = __float_as_uint(a.all);
+        }
+    };
+    // Fetches points until one is pending or none are left, then starts
+    // pending points of one job.  False when nothing could be started now.
+    auto start = [&]() -> bool {
+        while (more && !__ballot(pending >= 0)) {
+            const int fetch = min(fetch_max, max(fetch_min, (int)min((float)left * share, 64.f)));
+            unsigned long long b = 0;
+            if (lane == 0) b = atomicAdd(&cnt[DR_CNT_WORK + 16 * piece], (unsigned long long)fetch);
+            // the list index of the piece's f-th point (a piece: every eighth block of 256 points)
+            auto at = [&](long long f) { return ((f >> 8) * 8 + piece) * 256 + (f & 255); };
+            const long long f = (long long)__shfl(b, 0);
+            const long long i = at(f + lane);
+            if (lane < fetch && i < npoints) pending = list[i];
+            left = (npoints - at(f + fetch)) / 8;
+            if (at(f + fetch) >= npoints) {
+                piece = (piece + 1) & 7;
+                if (++tried == 8) more = false;
+            }
+        }
+        unsigned long long m = __ballot(pending >= 0);
+        if (!m) return false;
+        int pj = pending >= 0 ? pts[pending].job : 0;
+        int j0 = __shfl(pj, __ffsll((long long)m) - 1);
+        if (out0 + out1 == 0) job = __builtin_amdgcn_readfirstlane(j0);
+        if (j0 != job) return false;  // another job's points wait for this one's
+        // columns: on in the open half (from its start when none of its points
+        // has pending nodes), then in the other half when it has none
+        if ((open ? out1 : out0) == 0) used = 0;
+        const int room = 32 - used + ((open ? out0 : out1) == 0 ? 32 : 0);
+        if (room == 0) return false;
+        m = __ballot(pending >= 0 && pj == job);
+        int rank = __popcll(m & ((1ull << lane) - 1ull));
+        bool take = pending >= 0 && pj == job && rank < room;
+        uint32_t pt = (uint32_t)(open * 32 + used + rank) & 63u;
+        used += min(__popcll(m), room);
+        if (used > 32) {
+            open ^= 1;
+            used -= 32;
+        }
+        RootStack rs;
+        rs.sp = 0;
+        bool root = false;
+        if (take) {
+            const PointRec &p = pts[pending];
+            const DrJob &J = jobs[job];
+            EdgeTraversal T;
+            root = select_begin(J.S, J.c, p, T, rs) && rs.sp == 1 && !rs.e.empty();
+            if (root) {
+                auto c = [&](int k, float v) { C[k * 64 + pt] = __float_as_uint(v); };
+                c(0, p.sp.pos.x); c(1, p.sp.pos.y); c(2, p.sp.pos.z);
+                c(3, p.sp.fr.n.x); c(4, p.sp.fr.n.y); c(5, p.sp.fr.n.z);
+                c(6, T.B.hf.x.x); c(7, T.B.hf.x.y); c(8, T.B.hf.x.z);
+                c(9, T.B.hf.y.x); c(10, T.B.hf.y.y); c(11, T.B.hf.y.z);
+                c(12, T.B.hf.n.x); c(13, T.B.hf.n.y); c(14, T.B.hf.n.z);
+                c(15, T.B.lx); c(16, T.B.lz); c(17, T.B.e); c(18, T.B.dterm); c(19, T.B.slum);
+                c(20, p.cone_dir.x); c(21, p.cone_dir.y); c(22, p.cone_dir.z); c(23, p.cone_cos);
+                C[24 * 64 + pt] = (uint32_t)p.sid;
+                C[25 * 64 + pt] = (uint32_t)(p.sid >> 32);
+                C[26 * 64 + pt] = (T.directional ? 1u : 0u) | ((uint32_t)T.mode << 1) | ((uint32_t)p.b << 8);
+                C[27 * 64 + pt] = (uint32_t)pending;
+            }
+            pending = -1;
+        }
+        wave_lds_fence();
+        half_count(root, pt, out0, out1);
+        bool lf = root && rs.e.nprims() > 0;
+        add_leaf(lf, rs.e, rs.a, pt);
+        uint32_t x[SW];
+        pack(x, rs.e, rs.a, pt);
+        st.push(root && !lf, x, lane);
+        return true;
+    };
+
+    while (true) {
+        // new points when columns are free and lanes would stay idle
+        if ((used < 32 || out0 == 0 || out1 == 0) && st.blocks == 0 && st.n + __popcll(__ballot(has)) < 64) {
+            if (start()) continue;
+        }
+        // (a stack that is almost full is worked off by lane 0 alone)
+        const bool thr = st.throttled();
+        const bool on = !thr || lane == 0;
+        uint32_t x[SW];
+        if (st.pop(!has && on, x, lane)) {
+            for (int r = 0; r < SW; r++) cur[r] = x[r];
+            has = true;
+        }
+        if (!__ballot(has)) {
+            if (nleaf == 0) break;  // nothing pending, nothing to start
+            leaves(nleaf);
+            continue;
+        }
+        const bool run = has && on;
+        const uint32_t pt = cur[4];
+        TreeEntry c0, c1;
+        TreeAlt a0{0.f, 0.f}, a1{0.f, 0.f};
+        bool v0 = false, v1 = false;
+        if (run) {
+            const DrJob &J = jobs[job];
+            EdgeTraversal T;
+            SPoint sp;
+            load_point(pt, J, T, sp);
+            TreeEntry e{(int)cur[0], cur[1], cur[2], (int)cur[3]};
+            TreeAlt ea{0.f, 0.f};
+            if (LEARNED) ea = TreeAlt{__uint_as_float(cur[SW - 2]), __uint_as_float(cur[SW - 1])};
+            int k = et_expand(T, e, ea, J.S, sp, c0, a0, c1, a1);
+            // children whose bound is 0 take nothing
+            v0 = k > 0 && !c0.empty();
+            v1 = k > 1 && !c1.empty();
+            has = false;
+        }
+        {
+            const DrJob &J = jobs[job];
+            const int k = __popcll(__ballot(run));
+            if (J.S.stats && lane == 0) atomicAdd(&J.S.stats[5], (unsigned long long)k);
+        }
+        half_count(v0, pt, out0, out1);
+        half_count(v1, pt, out0, out1);
+        const bool l0 = v0 && c0.nprims() > 0, l1 = v1 && c1.nprims() > 0;
+        // the left child goes on in this lane, else the right one
+        bool p0 = v0 && !l0;
+        if (v1 && !l1) {
+            pack(cur, c1, a1, pt);
+            has = true;
+        } else if (p0) {
+            pack(cur, c0, a0, pt);
+            has = true;
+            p0 = false;
+        }
+        pack(x, c0, a0, pt);
+        st.push(p0, x, lane);
+        int d0 = 0, d1 = 0;
+        half_count(run, pt, d0, d1);
+        out0 -= d0;
+        out1 -= d1;
+        add_leaf(l0, c0, a0, pt);
+        add_leaf(l1, c1, a1, pt);
+        // a half may only wait for its last leaves
+        if (nleaf >= 16 && used == 32 && out0 > 0 && out1 > 0 && st.blocks == 0 && st.n + __popcll(__ballot(has)) < 64 &&
+             (more || __ballot(pending >= 0)))
+            leaves(nleaf);
     }
 }
 
@@ -823,49 +1082,76 @@ __global__ void k_intersect(DrSceneView S, const float *rays, long long n, int *
 // (0) uniform position on the segment, cosine lobe; (1) the LTC line sampler,
 // cosine lobe; (2) uniform, glossy; (3) the LTC line sampler, glossy.
 // out: per estimator the sum and the sum of squares (double).
-// dr_test_tree_stack: every lane runs `ops` random pushes and pops on the
-// selection kernel's LDS stack and on a plain array stack side by side (odd
-// waves with the alternative pmfs, even waves without); out[0] counts pops
-// that differ, out[1] the deepest stack reached.
-__global__ void __launch_bounds__(DR_BLOCK) k_tree_stack(long long ops, uint64_t seed, unsigned long long *out) {
-    __shared__ float s_stack[DR_LDS_STACK * DR_LDS_WORDS * DR_BLOCK];
-    LdsStack A;
-    A.lds = (DR_LDS float *)s_stack + threadIdx.x;
-    A.stride = DR_BLOCK;
-    A.clear();
-    PlainStack B;
-    B.clear();
-    Philox r;
-    philox_init(r, seed, 4, (uint64_t)blockIdx.x * blockDim.x + threadIdx.x, 0);
+// dr_test_tree_stack: every wave runs `ops` random pushes and pops of random
+// sets of its lanes on the selection kernel's wave stack, and keeps beside it
+// a plain array of what each position holds (position p: lane p % 64, element
+// p / 64 of its private array).  Odd waves carry 7 words per entry, even waves
+// 5; out[0] counts entries popped that differ, out[1] the deepest stack
+// reached, in entries per lane.
+template <int WORDS>
+DR_INLINE void tree_stack_run(long long ops, uint64_t seed, DR_LDS uint32_t *lds, unsigned long long *out) {
+    const int lane = (int)__lane_id();
+    const uint64_t wave = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
+    WaveStack<WORDS> A;
+    A.init(lds);
+    uint32_t ref[32];  // the operation that pushed the entry
+    int size = 0, deepest = 0;
     unsigned long long bad = 0;
-    int deepest = 0;
-    // with or without the alternative pmfs for a lane's whole run, as a walk
-    // of the selection kernel keeps its proposal mode: an entry pushed
-    // without them must not be popped with them (the stacks' slots for them
-    // would hold whatever private memory held before)
-    const bool alt = (threadIdx.x >> 6) & 1;
+    Philox rw, rl;
+    philox_init(rw, seed, 4, wave, 0);
+    philox_init(rl, seed, 4, wave * 64 + lane, 1);
+    auto word = [&](int p, uint32_t op, int r) { return (uint32_t)p * 0x9E3779B9u ^ op * 0x85EBCA6Bu ^ (uint32_t)r << 27; };
     for (long long k = 0; k < ops; k++) {
-        float u = philox_next(r);
-        bool push = B.size() == 0 || (B.size() < DR_TREE_STACK && u < 0.55f);
+        bool push = philox_next(rw) < 0.55f;
+        float share = philox_next(rw);
+        bool mine = philox_next(rl) < share;
+        uint32_t x[WORDS];
         if (push) {
-            int x = (int)(philox_next(r) * 16777216.f);
-            TreeEntry e{x - 8388608, __float_as_uint(philox_next(r)) ^ (uint32_t)x << 8,
-                        __float_as_uint(philox_next(r)) ^ (uint32_t)x << 11, x ^ 0x5555};
-            TreeAlt t{philox_next(r), philox_next(r)};
-            A.push(e, t, alt);
-            B.push(e, t, alt);
-            deepest = max(deepest, B.size());
+            // as many of the lanes as there is room for
+            unsigned long long m = __ballot(mine);
+            int rank = __popcll(m & ((1ull << lane) - 1ull));
+            mine = mine && size + rank < DR_WSTACK_CAP;
+            int n = __popcll(__ballot(mine));
+            for (int r = 0; r < WORDS; r++) x[r] = word(size + rank, (uint32_t)k, r);
+            A.push(mine, x, lane);
+            for (int i = 0; i < 32; i++) {
+                int p = i * 64 + lane;
+                if (p >= size && p < size + n) ref[i] = (uint32_t)k;
+            }
+            size += n;
         } else {
-            TreeAlt ta{0.f, 0.f}, tb{0.f, 0.f};
-            TreeEntry a = A.pop(ta, alt), b = B.pop(tb, alt);
-            if (a.code != b.code || a.cpmf != b.cpmf || a.apmf != b.apmf || a.off != b.off ||
-                (alt && (ta.cone != tb.cone || ta.all != tb.all)))
-                bad++;
+            unsigned long long m = __ballot(mine);
+            int rank = __popcll(m & ((1ull << lane) - 1ull));
+            bool got = A.pop(mine, x, lane);
+            int n = __popcll(__ballot(got));
+            // the plain array's entry at position size - 1 - rank: lanes get
+            // min(asked, stack) entries whenever the ring and one block hold
+            // enough, which they do
+            if (n != min(__popcll(m), size)) bad++;
+            int p = size - 1 - rank;
+            uint32_t mineref = 0;
+            for (int i = 0; i < 32; i++) {
+                int pp = i * 64 + lane;
+                if (pp >= size - n && pp < size) mineref = ref[i];
+            }
+            uint32_t op = __shfl(mineref, p & 63);
+            if (got)
+                for (int r = 0; r < WORDS; r++)
+                    if (x[r] != word(p, op, r)) bad++;
+            size -= n;
         }
-        if (A.size() != B.size()) bad++;
+        if (A.size() != size) bad++;
+        deepest = max(deepest, size / 64);
     }
     if (bad) atomicAdd(&out[0], bad);
     atomicMax(&out[1], (unsigned long long)deepest);
+}
+__global__ void __launch_bounds__(DR_BLOCK) k_tree_stack(long long ops, uint64_t seed, unsigned long long *out) {
+    __shared__ uint32_t s_stack[7 * DR_WSTACK_LDS * (DR_BLOCK / 64)];
+    const int w = threadIdx.x >> 6;
+    DR_LDS uint32_t *lds = (DR_LDS uint32_t *)s_stack + w * 7 * DR_WSTACK_LDS;
+    if (w & 1) tree_stack_run<7>(ops, seed, lds, out);
+    else tree_stack_run<5>(ops, seed, lds, out);
 }
 
 __global__ void __launch_bounds__(256) k_line_integral(long long n, uint64_t seed, double *out) {
@@ -1014,10 +1300,14 @@ struct Workspace {
     long long slot_cap = 0;
     EdgeEntry *q = nullptr;
     float4 *entry_dp = nullptr;
-    int *cont = nullptr;                     // queue entries left for the continuation launch
+    // queue entries left for the continuation launch (k_edge), and before it
+    // the list of the pass's points (k_sel_points: at most one per slot, and
+    // the queue has at least an entry per slot)
+    int *cont = nullptr;
     long long q_cap = 0;
-    // queue length, work counter, largest queue length, continuations,
-    // largest frontier end, largest leaf-list end (breadth-first selection)
+    // queue length, unused, largest queue length, continuations, largest
+    // frontier end, largest leaf-list end (breadth-first selection), points
+    // listed (DR_CNT_POINTS), unused; then the list's work counters
     unsigned long long *cnt = nullptr;
     unsigned long long *cnt_host = nullptr;  // pinned, 8 words
     SelPoint *spt = nullptr;                 // breadth-first selection: per point slot
@@ -1285,12 +1575,12 @@ static dr_status launch_check(const char *what) {
 
 // Resident workgroups of a kernel on this device (for persistent launches).
 template <class K>
-static long long resident_blocks(K kernel, long long &cache) {
+static long long resident_blocks(K kernel, long long &cache, int block = DR_BLOCK) {
     if (cache == 0) {
         int dev = 0, cus = 0, per_cu = 0;
         if (hipGetDevice(&dev) != hipSuccess ||
             hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-            hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, DR_BLOCK, 0) != hipSuccess || cus <= 0 ||
+            hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, block, 0) != hipSuccess || cus <= 0 ||
             per_cu <= 0) {
             cus = 256;
             per_cu = 2;
@@ -1314,6 +1604,8 @@ struct Plan {
     long long prim_blocks = 0, fwd_blocks = 0, max_slots = 0;
     int maxb = 1;
     int select_refill = 64;
+    int tree_nodes = 0;    // nodes of the largest edge tree of the adjoint jobs' scenes
+    bool learned = false;  // some adjoint job samples edges with the learned mixture
     int sel_depth = 0;  // deepest edge-tree node of the adjoint jobs' scenes (levels of the breadth-first selection)
     std::vector<std::pair<float *, size_t>> zero;  // buffers cleared first
     std::vector<unsigned long long> key;           // what a captured graph depends on
@@ -1364,6 +1656,8 @@ static dr_status build_plan(const dr_job *jobs, int n, const Tuning &tn, Plan &P
             P.zero.push_back({jb.grads, sc->hs.grad_size});
         }
         if (adj) P.maxb = std::max(P.maxb, bucket(jb.opts.max_bounces));
+        if (adj) P.tree_nodes = std::max(P.tree_nodes, (int)std::max(sc->hs.sil_nodes.size(), sc->hs.nrm_nodes.size()));
+        if (adj && (jb.opts.flags & DR_LEARNED_EDGES)) P.learned = true;
         if (adj) P.sel_depth = std::max(P.sel_depth, std::max(sc->hs.sil_depth, sc->hs.nrm_depth));
         P.jobs.push_back(dj);
         unsigned long long k[] = {(unsigned long long)(uintptr_t)sc, sc->serial, (unsigned long long)sc->hs.grad_size,
@@ -1439,6 +1733,7 @@ static dr_status build_plan(const dr_job *jobs, int n, const Tuning &tn, Plan &P
     // deeper trees are walked depth first
     P.select_refill = tn.select_refill == 0 && P.sel_depth > 62 ? 64 : tn.select_refill;
     P.key.push_back((unsigned long long)P.sel_depth);
+    P.key.push_back((unsigned long long)P.tree_nodes);
     P.key.push_back((unsigned long long)tn.pass_samples);
     P.key.push_back((unsigned long long)tn.min_threads);
     P.key.push_back((unsigned long long)tn.select_refill);
@@ -1457,7 +1752,7 @@ static dr_status ensure_workspace(Workspace &w, const Plan &P) {
 }
 static dr_status ensure_workspace_(Workspace &w, const Plan &P) {
     if (!w.cnt) {
-        if (hipMalloc((void **)&w.cnt, 8 * sizeof(unsigned long long)) != hipSuccess ||
+        if (hipMalloc((void **)&w.cnt, DR_CNT_WORDS * sizeof(unsigned long long)) != hipSuccess ||
             hipHostMalloc((void **)&w.cnt_host, 8 * sizeof(unsigned long long), hipHostMallocDefault) != hipSuccess)
             return fail(DR_ERROR_OUT_OF_MEMORY, "adjoint counters");
     }
@@ -1545,7 +1840,7 @@ static dr_status grow_queue(Workspace &w, long long n) {
     return DR_OK;
 }
 
-static long long g_select_blocks = 0, g_edge_blocks[4] = {0, 0, 0, 0}, g_shade_blocks[4] = {0, 0, 0, 0};
+static long long g_select_blocks[2] = {0, 0}, g_edge_blocks[4] = {0, 0, 0, 0}, g_shade_blocks[4] = {0, 0, 0, 0};
 static long long g_sel_blocks[3] = {0, 0, 0};
 
 // All launches of a plan, stream-ordered, without host synchronisation (so
@@ -1584,6 +1879,29 @@ static dr_status grow_overflowed(Workspace &w, long long qlen, bool bfs, bool &g
     return DR_OK;
 }
 
+// The depth-first selection of the points f in [f0, f1): one resident grid of
+// one-wave workgroups.  A wave fetches at least 4 slots at a time, more where
+// the trees are so small that no point's walk is long: fetches of 4 cost the
+// single triangle (11 nodes) 0.6 ms a render in contended atomics and starts
+// of few points, and 64 cost a 64 x 64 heightfield (24 k nodes) 4 ms of 15 in
+// waves that finish late.
+static void launch_select(const Plan &P, const Workspace &w, long long nslots, int maxb, int fetch_max, long long f0,
+                          long long f1, hipStream_t hs) {
+    long long waves = P.learned ? resident_blocks(k_select<true>, g_select_blocks[1], 64)
+                                : resident_blocks(k_select<false>, g_select_blocks[0], 64);
+    long long n = f1 - f0;
+    int fetch_min = std::min(fetch_max, std::max(4, std::min(64, 4096 / std::max(1, P.tree_nodes))));
+    unsigned grid = (unsigned)std::min<long long>(waves, (n + fetch_min - 1) / fetch_min);
+    const int per_block = DR_BLOCK * DR_LIST_PER_THREAD;
+    k_fill<<<1, 256, 0, hs>>>((float *)(w.cnt + DR_CNT_POINTS), 2 * (DR_CNT_WORDS - DR_CNT_POINTS), 0.f);
+    k_sel_points<<<(unsigned)((n + per_block - 1) / per_block), DR_BLOCK, 0, hs>>>(nslots, maxb, w.pts, w.cont, w.cnt,
+                                                                                  w.counts, f0, f1);
+    if (P.learned)
+        k_select<true><<<grid, 64, 0, hs>>>(w.jobs, w.cont, w.pts, w.q, w.cnt, w.q_cap, w.counts, fetch_min, fetch_max);
+    else
+        k_select<false><<<grid, 64, 0, hs>>>(w.jobs, w.cont, w.pts, w.q, w.cnt, w.q_cap, w.counts, fetch_min, fetch_max);
+}
+
 template <class Launch>
 static dr_status settle_selection(Workspace &w, hipStream_t hs, bool bfs, Launch &&select) {
     for (int attempt = 0; attempt < 8; attempt++) {
@@ -1620,7 +1938,7 @@ static dr_status enqueue(const Plan &P, Workspace &w, Timing *tm, hipStream_t hs
         if (!ps.edges) continue;
         k_fill<<<1024, 256, 0, hs>>>(w.pt_dp, (size_t)ps.nslots * 3, 0.f);
         k_fill_i<<<1024, 256, 0, hs>>>(w.pt_lastj, (size_t)ps.nslots, -1);
-        k_fill<<<1, 64, 0, hs>>>((float *)w.cnt, 4, 0.f);        // queue length, work counter
+        k_fill<<<1, 64, 0, hs>>>((float *)w.cnt, 4, 0.f);        // queue length
         k_fill<<<1, 64, 0, hs>>>((float *)(w.cnt + 3), 2, 0.f);  // continuations
         auto select = [&]() {
             LaunchTimer t(tm, TK_SELECT, hs);
@@ -1638,9 +1956,7 @@ static dr_status enqueue(const Plan &P, Workspace &w, Timing *tm, hipStream_t hs
                 k_sel_leaves<<<(unsigned)b2, DR_BLOCK, 0, hs>>>(w.jobs, w.spt, w.lv, w.lvl + DR_SEL_LEAVES, w.l_cap,
                                                                 w.q, w.cnt, w.q_cap, w.counts);
             } else {
-                long long blocks = std::min<long long>(grid_of(ps.nslots), resident_blocks(k_select, g_select_blocks));
-                k_select<<<(unsigned)blocks, DR_BLOCK, 0, hs>>>(w.jobs, ps.nslots, MAXB, w.pts, w.q, w.cnt, w.q_cap,
-                                                                w.counts, P.select_refill, 0ll, ps.nslots);
+                launch_select(P, w, ps.nslots, MAXB, P.select_refill, 0ll, ps.nslots, hs);
             }
         };
         select();
@@ -1833,13 +2149,10 @@ static dr_status run_noalloc(const Plan &P, Workspace &w, hipStream_t hs) {
         long long part = per > 0.0 ? std::max(1ll, (long long)(0.9 * (double)w.q_cap / per)) : ps.nslots;
         for (long long f0 = 0; f0 < ps.nslots;) {
             long long f1 = std::min(ps.nslots, f0 + part);
-            k_fill<<<1, 64, 0, hs>>>((float *)w.cnt, 2 * 2, 0.f);       // queue length, work counter
+            k_fill<<<1, 64, 0, hs>>>((float *)w.cnt, 2 * 2, 0.f);       // queue length
             k_fill<<<1, 64, 0, hs>>>((float *)(w.cnt + 3), 2, 0.f);     // continuations
-            long long blocks = std::min<long long>(grid_of(f1 - f0), resident_blocks(k_select, g_select_blocks));
             // (the depth-first selection: its working set fits the array)
-            k_select<<<(unsigned)blocks, DR_BLOCK, 0, hs>>>(w.jobs, ps.nslots, MAXB, w.pts, w.q, w.cnt, w.q_cap,
-                                                            w.counts, P.select_refill > 0 ? P.select_refill : 64,
-                                                            f0, f1);
+            launch_select(P, w, ps.nslots, MAXB, P.select_refill > 0 ? P.select_refill : 64, f0, f1, hs);
             unsigned long long len = 0;
             if (hipMemcpyAsync(&len, w.cnt, sizeof(len), hipMemcpyDeviceToHost, hs) != hipSuccess ||
                 hipStreamSynchronize(hs) != hipSuccess)
@@ -2331,7 +2644,7 @@ dr_status dr_render_adjoint_noalloc(dr_scene *s, const dr_render_options *o, con
         return fail(DR_ERROR_UNSUPPORTED, "the render needs more passes than the allocation-free tables hold");
     Carver c{(char *)base, 0, DR_NOALLOC_BYTES};
     Workspace w;
-    w.cnt = c.take<unsigned long long>(4);
+    w.cnt = c.take<unsigned long long>(DR_CNT_WORDS);
     w.jobs = c.take<DrJob>(1);
     w.ranges = c.take<DrRange>(DR_NOALLOC_MAX_RANGES);
     long long slots = std::max<long long>(P.max_slots, 1);
