@@ -49,43 +49,25 @@ struct Cone {
 // Geometric Tools Engine, David Eberly, Geometric Tools LLC, distributed
 // under the Boost Software License 1.0.  Box corners in CCW order for each
 // of the 27 apex regions; geometric data that must match the reference.
-__constant__ static const signed char kConePolyN[27] = {6, 6, 6, 6, 4, 6, 6, 6, 6, 6, 4, 6, 4, 0,
-                                                         4, 6, 4, 6, 6, 6, 6, 6, 4, 6, 6, 6, 6};
-__constant__ static const signed char kConePolyIdx[27][6] = {
-    {1, 5, 4, 6, 2, 3}, {0, 2, 3, 1, 5, 4}, {0, 2, 3, 7, 5, 4}, {0, 4, 6, 2, 3, 1}, {0, 2, 3, 1, 0, 0},
-    {0, 2, 3, 7, 5, 1}, {0, 4, 6, 7, 3, 1}, {0, 2, 6, 7, 3, 1}, {0, 2, 6, 7, 5, 1}, {0, 1, 5, 4, 6, 2},
-    {0, 1, 5, 4, 0, 0}, {0, 1, 3, 7, 5, 4}, {0, 4, 6, 2, 0, 0}, {0, 0, 0, 0, 0, 0}, {1, 3, 7, 5, 0, 0},
-    {0, 4, 6, 7, 3, 2}, {2, 6, 7, 3, 0, 0}, {1, 3, 2, 6, 7, 5}, {0, 1, 5, 7, 6, 2}, {0, 1, 5, 7, 6, 4},
-    {0, 1, 3, 7, 6, 4}, {0, 4, 5, 7, 6, 2}, {4, 5, 7, 6, 0, 0}, {1, 3, 7, 6, 4, 5}, {0, 4, 5, 7, 3, 2},
-    {2, 6, 4, 5, 7, 3}, {1, 3, 2, 6, 4, 5}};
+// Corner i of a region's polygon is 3 bits at 3 i (bit 0, 1, 2 of a corner: on
+// the high side in x, y, z); bit 18: six corners instead of four (region 13,
+// the apex inside the box, has none).
+__constant__ static const uint32_t kConePoly[27] = {
+    0x5ad29, 0x652d0, 0x65ed0, 0x4b5a0, 0x002d0, 0x4ded0,
+    0x4bfa0, 0x4bf90, 0x4df90, 0x56948, 0x00948, 0x65ec8,
+    0x005a0, 0x00000, 0x00bd9, 0x53fa0, 0x007f2, 0x6fc99,
+    0x56f48, 0x66f48, 0x66ec8, 0x56f60, 0x00dec, 0x6cdd9,
+    0x53f60, 0x5fb32, 0x6cc99};
 
 // component k (0, 1, 2) of v, by value (no runtime indexing of a vector)
 DR_INLINE float comp(F3 v, int k) { return k == 0 ? v.x : (k == 1 ? v.y : v.z); }
 
-DR_INLINE bool cone_edge_test(F3 D, float c2, F3 maxX, F3 maxPmV, float maxSqrLen, float maxDd, F3 CmV, int jA,
-                              int jB, float flip, bool &decided) {
-    int jDiff = jB - jA;
-    float s = jDiff > 0 ? 1.f : -1.f;
-    int k0 = abs(jDiff) >> 1;
-    float fder = flip * s * (comp(D, k0) * maxSqrLen - maxDd * comp(maxPmV, k0));
-    decided = fder > 0;
-    if (!decided) return false;
-    int k1 = (k0 + 1) % 3, k2 = (k1 + 1) % 3;
-    float p1 = comp(maxPmV, k1), p2 = comp(maxPmV, k2);
-    float d1 = comp(D, k1), d2 = comp(D, k2);
-    float numer = p1 * p1 + p2 * p2;
-    float denom = d1 * p1 + d2 * p2;
-    float m0 = numer * comp(D, k0);
-    float m1 = denom * (comp(maxX, k1) + comp(CmV, k1));
-    float m2 = denom * (comp(maxX, k2) + comp(CmV, k2));
-    // M has m0 at k0, m1 at k1, m2 at k2
-    F3 M = F3{k0 == 0 ? m0 : (k1 == 0 ? m1 : m2), k0 == 1 ? m0 : (k1 == 1 ? m1 : m2),
-              k0 == 2 ? m0 : (k1 == 2 ? m1 : m2)};
-    float DdM = dot(D, M);
-    if (DdM * DdM - c2 * dot(M, M) > 0) return true;
-    return s * (d1 * p2 - d2 * p1) <= 0;
-}
-
+// The corners' table entry is read once, the polygon walk keeps only the best
+// corner's number and ratio, and the two edges at it share one copy of the
+// edge test: the walk is the longest part of expanding a node, and the wave
+// runs it whenever one of its lanes does.  (With the lighter node bound, the
+// silhouette test below and one multiply per Philox product: 31.6 -> 24.2 ms a
+// selection pass of the 512 x 512 heightfield.)
 DR_INLINE bool aabb_cone_intersect(const float *lo, const float *hi, const Cone &cone) {
     if (cone.cos_angle <= 0.f) return true;
     F3 center = 0.5f * (F3{lo[0], lo[1], lo[2]} + F3{hi[0], hi[1], hi[2]});
@@ -100,35 +82,68 @@ DR_INLINE bool aabb_cone_intersect(const float *lo, const float *hi, const Cone 
     int iz = CmV.z < -ext.z ? 2 : (CmV.z > ext.z ? 0 : 1);
     int lookup = ix + 3 * iy + 9 * iz;
     if (lookup == 13) return true;
-    int np = kConePolyN[lookup];
+    const uint32_t poly = kConePoly[lookup];
+    const bool six = (poly >> 18) != 0;
     float c2 = cone.cos_angle * cone.cos_angle;
-    int iMax = -1, jMax = -1;
-    float maxSqrDd = 0.f, maxSqrLen = 0.f, maxDd = 0.f;
-    F3 maxX = F3{0.f, 0.f, 0.f}, maxPmV = F3{0.f, 0.f, 0.f};
-    for (int i = 0; i < np; i++) {
-        int j = kConePolyIdx[lookup][i];
-        F3 X = F3{(j & 1) ? ext.x : -ext.x, (j & 2) ? ext.y : -ext.y, (j & 4) ? ext.z : -ext.z};
+    // corner j relative to the box's centre (extents are not negative)
+    auto corner = [&](uint32_t j) {
+        return F3{copysignf(ext.x, __uint_as_float(~j << 31)), copysignf(ext.y, __uint_as_float(~j << 30)),
+                  copysignf(ext.z, __uint_as_float(~j << 29))};
+    };
+    bool inside = false;
+    int iMax = -1;
+    float maxSqrDd = 0.f, maxSqrLen = 0.f;
+#pragma unroll
+    for (int i = 0; i < 6; i++) {
+        if (i >= 4 && !six) continue;
+        F3 X = corner(poly >> (3 * i));
         float Dd = dot(D, X) + DdCmV;
-        if (Dd > 0) {
-            F3 PmV = X + CmV;
-            float sqrDd = Dd * Dd;
-            float sqrLen = dot(PmV, PmV);
-            if (sqrDd - c2 * sqrLen > 0) return true;
-            if (iMax == -1 || sqrDd * maxSqrLen > maxSqrDd * sqrLen) {
-                iMax = i; jMax = j;
-                maxSqrDd = sqrDd; maxSqrLen = sqrLen; maxDd = Dd; maxX = X; maxPmV = PmV;
-            }
-        }
+        F3 PmV = X + CmV;
+        float sqrDd = Dd * Dd;
+        float sqrLen = dot(PmV, PmV);
+        bool front = Dd > 0;
+        inside |= front && sqrDd - c2 * sqrLen > 0;
+        bool better = front && (iMax == -1 || sqrDd * maxSqrLen > maxSqrDd * sqrLen);
+        iMax = better ? i : iMax;
+        maxSqrDd = better ? sqrDd : maxSqrDd;
+        maxSqrLen = better ? sqrLen : maxSqrLen;
     }
+    if (inside) return true;
     if (iMax == -1) return false;
-    int jNext = kConePolyIdx[lookup][iMax < np - 1 ? iMax + 1 : 0];
-    bool decided;
-    bool r = cone_edge_test(D, c2, maxX, maxPmV, maxSqrLen, maxDd, CmV, jMax, jNext, 1.f, decided);
-    if (decided) return r;
-    int jPrev = kConePolyIdx[lookup][iMax > 0 ? iMax - 1 : np - 1];
-    r = cone_edge_test(D, c2, maxX, maxPmV, maxSqrLen, maxDd, CmV, jPrev, jMax, -1.f, decided);
-    if (decided) return r;
-    return false;
+    const int last = six ? 5 : 3;
+    const uint32_t jM = poly >> (3 * iMax);
+    const int jMax = (int)(jM & 7u);
+    const int jNext = (int)((poly >> (3 * (iMax < last ? iMax + 1 : 0))) & 7u);
+    const int jPrev = (int)((poly >> (3 * (iMax > 0 ? iMax - 1 : last))) & 7u);
+    const F3 maxX = corner(jM), maxPmV = maxX + CmV;
+    const float maxDd = dot(D, maxX) + DdCmV;
+    // the derivative along the edge to the next corner, then along the one
+    // from the previous corner: the first that grows decides
+    int jDiff = jNext - jMax;
+    int k0 = abs(jDiff) >> 1;
+    float s = jDiff > 0 ? 1.f : -1.f;
+    float fder = s * (comp(D, k0) * maxSqrLen - maxDd * comp(maxPmV, k0));
+    if (!(fder > 0)) {
+        jDiff = jMax - jPrev;
+        k0 = abs(jDiff) >> 1;
+        s = jDiff > 0 ? 1.f : -1.f;
+        fder = -s * (comp(D, k0) * maxSqrLen - maxDd * comp(maxPmV, k0));
+        if (!(fder > 0)) return false;
+    }
+    int k1 = k0 == 2 ? 0 : k0 + 1, k2 = k0 == 0 ? 2 : k0 - 1;
+    float p1 = comp(maxPmV, k1), p2 = comp(maxPmV, k2);
+    float d1 = comp(D, k1), d2 = comp(D, k2);
+    float numer = p1 * p1 + p2 * p2;
+    float denom = d1 * p1 + d2 * p2;
+    float m0 = numer * comp(D, k0);
+    float m1 = denom * (comp(maxX, k1) + comp(CmV, k1));
+    float m2 = denom * (comp(maxX, k2) + comp(CmV, k2));
+    // M has m0 at k0, m1 at k1, m2 at k2
+    F3 M = F3{k0 == 0 ? m0 : (k1 == 0 ? m1 : m2), k0 == 1 ? m0 : (k1 == 1 ? m1 : m2),
+              k0 == 2 ? m0 : (k1 == 2 ? m1 : m2)};
+    float DdM = dot(D, M);
+    if (DdM * DdM - c2 * dot(M, M) > 0) return true;
+    return s * (d1 * p2 - d2 * p1) <= 0;
 }
 
 DR_INLINE float min_sq_bound(float lo, float hi) {
@@ -190,8 +205,8 @@ DR_INLINE float bsdf_bound(const DrEdgeNode &node, const SPoint &sp, const Bound
         // the box in the frame around wi: per local axis j, base + extents
         const Frame &f = B.hf;
         F3 l0 = to_local(f, b);
-        F3 ax = to_local(f, F3{ext.x, 0.f, 0.f}), ay = to_local(f, F3{0.f, ext.y, 0.f}),
-           az = to_local(f, F3{0.f, 0.f, ext.z});
+        F3 ax = F3{ext.x * f.x.x, ext.x * f.y.x, ext.x * f.n.x}, ay = F3{ext.y * f.x.y, ext.y * f.y.y, ext.y * f.n.y},
+           az = F3{ext.z * f.x.z, ext.z * f.y.z, ext.z * f.n.z};
         float blo[3], bhi[3];
         blo[0] = l0.x + fminf(ax.x, 0.f) + fminf(ay.x, 0.f) + fminf(az.x, 0.f);
         bhi[0] = l0.x + fmaxf(ax.x, 0.f) + fmaxf(ay.x, 0.f) + fmaxf(az.x, 0.f);
@@ -237,19 +252,35 @@ DR_INLINE float bsdf_bound(const DrEdgeNode &node, const SPoint &sp, const Bound
 // difference lies in [0, pi/2], so the test is sin(acos(-d.axis)) >=
 // cos(angle + va), which also holds whenever angle + va >= pi/2.  The same
 // verdicts as the angles' up to rounding at the boundary.
+// The verdict is first taken from the hardware's reciprocal and square root
+// (errors of a few 1e-7); only where both sides are too close for that (about
+// one node in a thousand) do the correctly rounded quotients decide, so the
+// verdict is theirs always.
 DR_INLINE bool contains_silhouette(const DrEdgeNode &n, F3 p) {
     F3 lo = F3{n.lo[0], n.lo[1], n.lo[2]}, hi = F3{n.hi[0], n.hi[1], n.hi[2]};
     F3 c = (lo + hi) / 2.f;
-    float r = length(hi - c);
     F3 d = c - p;
     float len2 = length_sq(d);
     float len = approx_sqrt(len2);
-    float tv = r / len;
-    if (tv >= 1.f) return true;
-    float ca = -dot(d, F3{n.axis[0], n.axis[1], n.axis[2]}) / len;
-    float s_ang = approx_sqrt(fmaxf(1.f - ca * ca, 0.f));
+    float r2 = length_sq(hi - c);
+    float da = -dot(d, F3{n.axis[0], n.axis[1], n.axis[2]});
     float cA = n.cos_angle, sA = approx_sqrt(fmaxf(1.f - cA * cA, 0.f));
-    // cos(angle + va) = (cos(angle) - sin(angle) tv) / sqrt(1 + tv^2)
+    {
+        float il = approx_rcp(len);
+        float tv = approx_sqrt(r2) * il, ca = da * il;
+        float s2 = 1.f - ca * ca;
+        // cos(angle + va) = (cos(angle) - sin(angle) tv) / sqrt(1 + tv^2)
+        float diff = approx_sqrt(fmaxf(s2, 0.f)) * approx_sqrt(1.f + tv * tv) - (cA - sA * tv);
+        // an error of 5e-7 in s2 is one of 8e-6 in its root above 1e-3, and of
+        // at most 8e-4 below
+        float margin = s2 > 1e-3f ? 5e-5f : 4e-3f;
+        if (tv > 1.0001f) return true;
+        if (tv < 0.9999f && fabsf(diff) > margin) return diff > 0.f;
+    }
+    float tv = sqrtf(r2) / len;
+    if (tv >= 1.f) return true;
+    float ca = da / len;
+    float s_ang = approx_sqrt(fmaxf(1.f - ca * ca, 0.f));
     return s_ang * approx_sqrt(1.f + tv * tv) >= cA - sA * tv;
 }
 
@@ -325,11 +356,11 @@ struct TreeAlt {
 // pop.  Every lane of the wave calls push and pop together.  When all blocks
 // nearly in use, throttled() asks the caller to let lane 0 alone pop, expand
 // and push: a depth-first walk adds at most one entry per tree level, for which
-// there is room beside one push of all lanes.
+// there is room beside two pushes of all lanes.
 #define DR_WSTACK_LDS 128
 #define DR_WSTACK_BLOCKS 30
 #define DR_WSTACK_CAP (DR_WSTACK_BLOCKS * 64 + DR_WSTACK_LDS)  // 32 entries per lane
-static_assert(DR_TREE_STACK <= 32, "throttled() leaves room for 32 entries of one lane's walk");
+static_assert(DR_TREE_STACK + 2 <= 40, "throttled() leaves room for one lane's walk");
 DR_INLINE void wave_lds_fence() {
 #if defined(__HIP_DEVICE_COMPILE__)
     // orders the wave's LDS accesses for the compiler (the hardware runs a
@@ -349,7 +380,7 @@ struct WaveStack {
         n = base = blocks = 0;
     }
     DR_INLINE int size() const { return n + 64 * blocks; }
-    DR_INLINE bool throttled() const { return size() > DR_WSTACK_CAP - 64 - 32; }
+    DR_INLINE bool throttled() const { return size() > DR_WSTACK_CAP - 2 * 64 - 40; }
     // lanes with `have` push their entry, lower lanes below higher ones
     DR_INLINE void push(bool have, const uint32_t *x, int lane) {
         unsigned long long m = __ballot(have);
@@ -509,13 +540,23 @@ DR_INLINE void et_leaf_edge(const EdgeTraversal &T, const TreeEntry &e, TreeAlt 
     if (mask & 2) emit(scale * all_pmf / den, T.directional, e.off + i, DR_ORD_ALL_PASS | (e.off + i));
 }
 
+// Whether the cone pass can still reach the node's subtree (its own mask bit
+// or a nonzero pmf of either proposal); otherwise every quantity the cone
+// tests feed is multiplied by zero.  Children of a node without it have none
+// either.
+DR_INLINE bool et_need_cone(const TreeEntry &e, TreeAlt ea) {
+    return (e.mask() & 1) || e.cone_pmf() != 0.f || ea.cone != 0.f;
+}
+
 // An interior node: the children the passes go on to, at most two, in the
 // order a depth-first walk pushes them (right, then left).  Returns how
-// many (c0 first, then c1).
+// many (c0 first, then c1).  CONE false: for nodes without et_need_cone, the
+// same result without the cone tests' code.
+template <bool CONE = true>
 DR_INLINE int et_expand(EdgeTraversal &T, const TreeEntry &e, TreeAlt ea, const DrSceneView &S, const SPoint &sp,
                         TreeEntry &c0, TreeAlt &a0, TreeEntry &c1, TreeAlt &a1) {
-    const int ni = e.node(), mask = e.mask();
-    const float cone_pmf = e.cone_pmf(), all_pmf = e.all_pmf();
+    const int ni = e.node(), mask = CONE ? e.mask() : e.mask() & 2;
+    const float cone_pmf = CONE ? e.cone_pmf() : 0.f, all_pmf = e.all_pmf();
     int li = ni + 1, ri = e.off;
     const DrEdgeNode L = gptr(T.nodes)[li], R = gptr(T.nodes)[ri];
     bool all_split = e.split_all();
@@ -541,10 +582,7 @@ DR_INLINE int et_expand(EdgeTraversal &T, const TreeEntry &e, TreeAlt ea, const 
         }
     }
     if (il + ir <= 1e-10f) return 0;
-    // the cone tests only matter while the cone pass can still reach the
-    // node's subtree (its own mask bit or a nonzero pmf of either proposal);
-    // otherwise every quantity they feed is multiplied by zero
-    bool need_cone = (mask & 1) || cone_pmf != 0.f || (T.mode != 0 && ea.cone != 0.f);
+    const bool need_cone = CONE && et_need_cone(e, ea);
     bool lhc = need_cone && aabb_cone_intersect(L.lo, L.hi, T.cone);
     bool rhc = need_cone && aabb_cone_intersect(R.lo, R.hi, T.cone);
     bool cone_split = all_split || (lhc && rhc && lcs && rcs && T.cone.cos_angle > 0.95f);

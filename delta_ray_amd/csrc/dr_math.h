@@ -275,8 +275,11 @@ DR_INLINE void philox_refill(Philox &r) {
     uint32_t a = r.k0, b = r.k1;
 #pragma unroll
     for (int i = 0; i < 10; i++) {
-        uint32_t lo0 = 0xD2511F53u * x0, hi0 = __umulhi(0xD2511F53u, x0);
-        uint32_t lo1 = 0xCD9E8D57u * x2, hi1 = __umulhi(0xCD9E8D57u, x2);
+        // (one 64-bit multiply-add for both words of a product: 32-bit integer
+        // multiplies run at a quarter of the vector rate)
+        uint64_t m0 = (uint64_t)0xD2511F53u * x0, m1 = (uint64_t)0xCD9E8D57u * x2;
+        uint32_t lo0 = (uint32_t)m0, hi0 = (uint32_t)(m0 >> 32);
+        uint32_t lo1 = (uint32_t)m1, hi1 = (uint32_t)(m1 >> 32);
         uint32_t n0 = hi1 ^ x1 ^ a;
         uint32_t n2 = hi0 ^ x3 ^ b;
         x0 = n0; x1 = lo1; x2 = n2; x3 = lo0;

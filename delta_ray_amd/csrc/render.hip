@@ -7,7 +7,8 @@
 //   pipeline over batches of pixel samples:
 //     k_path    camera path + radiance + interior adjoint; stores one
 //               PointRec per (sample, bounce) shading point
-//     k_select  edge-tree traversal per shading point -> queue of edges
+//     k_sel_points, k_select  list of the shading points; edge-tree traversal
+//               of a wave's points together -> queue of edges
 //     k_edge    thread = one selected edge: secondary edge sample, vertex
 //               gradients, Dirac position derivative dp of its point
 //     k_dp_last keeps the last dp per point (set_adjoint overwrite)
@@ -33,6 +34,7 @@
 #include <cstring>
 #include <new>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #define DR_BLOCK 256
@@ -477,18 +479,25 @@ __global__ void __launch_bounds__(DR_BLOCK) k_sel_points(long long nslots, int m
 // length of a point's walk varies by two orders of magnitude and more (a point
 // inside many node boxes splits at every level), so a lane per point leaves
 // most of a wave waiting for its longest walk (27 of 64 lanes active), and a
-// small render waits for single lanes that walk alone.  Here the pending nodes
-// of up to 64 points sit in one stack per wave (WaveStack): every iteration
-// each lane expands one node, whichever point it belongs to, keeps one of its
-// interior children as its next node, and idle lanes take theirs from the
-// stack.  A node's draws are keyed by point and node, so the selected edges do
-// not depend on the order.
+// small render waits for single lanes that walk alone (such a kernel took
+// 27.5 ms for 128 x 128 x 4 samples of a 64 x 64 heightfield and 55.7 ms for a
+// 4.2 M sample pass of the 128 x 128 one; this one took 4.4 ms and 36 ms in its
+// place).  Here the pending nodes of up to 64 points sit in one stack per wave
+// (WaveStack): every iteration each lane takes one node from the top,
+// whichever point it belongs to, and pushes its children.  A node's draws are keyed by point and
+// node, so the selected edges do not depend on the order.
 //   * Points: what expanding and testing need of a point (SEL_WORDS words, from
 //     its PointRec and bound_ctx) lies in LDS, a column per point.  A wave
 //     holds two halves of 32 points; a half whose nodes are all done takes new
 //     points while the other half's walk goes on, and points are added whenever
 //     lanes would stay idle, so lanes run dry only at the end of the launch.  The points of a wave belong to one job at a time
 //     (scene pointers and random key stay in scalar registers).
+//   * Two stacks: nodes the cone pass can still reach (et_need_cone: a third of
+//     a heightfield's nodes), whose expansion walks a box's silhouette polygon
+//     for each child, and the others, whose expansion has no such code.  A
+//     wave's lanes all expand nodes of one kind; mixed, the third of the lanes
+//     with cone tests kept the others waiting for nearly half of the
+//     instructions.
 //   * Leaves wait in a list in LDS until there are 64 of them, so the
 //     silhouette test runs on full waves and a wave's selected edges are
 //     appended to the queue with one atomic.
@@ -498,25 +507,27 @@ __global__ void __launch_bounds__(DR_BLOCK) k_sel_points(long long nslots, int m
 // (workgroups go to the XCDs in turn), each with its own counter in its own
 // cache line, so that fetches do not queue up at one address; a wave whose
 // piece is used up goes on to the next one.  A fetch takes a fortieth of an even share
-// of what is left of the piece, between fetch_min and 64 points: neighbouring
+// of what is left of the piece, between fetch_min and 16 points: neighbouring
 // points are heavy together (some 20 times the mean walk), and a wave that
 // took many of them last would finish long after the others (with 64 points
-// at any time the waves of the 512 x 512 heightfield ran 59 % of the launch).
+// at any time the waves of the 512 x 512 heightfield ran 59 % of the launch;
+// at most 64, 32, 16, 8 and 4 at a time: 294, 297, 287, 289 and 290 ms a render).
 #define SEL_WORDS 28
 template <bool LEARNED>
 __global__ void __launch_bounds__(64)
 k_select(const DrJob *__restrict__ jobs, const int *list, const PointRec *pts, EdgeEntry *q, unsigned long long *cnt,
          long long cap, int *counts, int fetch_min, int fetch_max) {
-    constexpr int SW = LEARNED ? 7 : 5, LW = LEARNED ? 6 : 4;
+    constexpr int SW = LEARNED ? 6 : 4;  // words of an entry
     constexpr int LEAVES = 128;  // 63 waiting and the 64 a round adds
     __shared__ uint32_t s_point[SEL_WORDS * 64];
-    __shared__ uint32_t s_stack[SW * DR_WSTACK_LDS];
-    __shared__ uint32_t s_leaf[LW * LEAVES];
+    __shared__ uint32_t s_stack[2][SW * DR_WSTACK_LDS];
+    __shared__ uint32_t s_leaf[SW * LEAVES];
     DR_LDS uint32_t *C = (DR_LDS uint32_t *)s_point, *LF = (DR_LDS uint32_t *)s_leaf;
     const long long npoints = (long long)cnt[DR_CNT_POINTS];
     const int lane = (int)__lane_id();
-    WaveStack<SW> st;
-    st.init((DR_LDS uint32_t *)s_stack);
+    WaveStack<SW> cst, ast;  // nodes with and without et_need_cone
+    cst.init((DR_LDS uint32_t *)s_stack[0]);
+    ast.init((DR_LDS uint32_t *)s_stack[1]);
     int nleaf = 0, leaf0 = 0;  // leaves waiting (a ring), the oldest
     int out0 = 0, out1 = 0; // nodes and leaves pending of either half's points
     int open = 0, used = 0; // the half that takes new points, its columns taken
@@ -526,8 +537,6 @@ k_select(const DrJob *__restrict__ jobs, const int *list, const PointRec *pts, E
     long long left = npoints / 8;                  // points of the piece left at this wave's last fetch
     const float share = 8.f / (40.f * (float)gridDim.x);
     long long pending = -1; // a fetched point not started yet
-    bool has = false;       // this lane holds a node
-    uint32_t cur[SW] = {};  // TreeEntry, point [, TreeAlt]
 
     auto half_count = [&](bool v, uint32_t pt, int &o0, int &o1) {
         int a = __popcll(__ballot(v)), b = __popcll(__ballot(v && pt >= 32));
@@ -583,7 +592,7 @@ k_select(const DrJob *__restrict__ jobs, const int *list, const PointRec *pts, E
             uint32_t a = LF[2 * LEAVES + i], o = LF[3 * LEAVES + i];
             te = TreeEntry{(int)LF[i], LF[LEAVES + i], a & 0x7fffffffu, (int)(o & 0x7ffffffu)};
             pt = (o >> 27) | (a >> 31) << 5;
-            if (LEARNED) ta = TreeAlt{__uint_as_float(LF[(LW - 2) * LEAVES + i]), __uint_as_float(LF[(LW - 1) * LEAVES + i])};
+            if (LEARNED) ta = TreeAlt{__uint_as_float(LF[(SW - 2) * LEAVES + i]), __uint_as_float(LF[(SW - 1) * LEAVES + i])};
             nprims = te.nprims();
             sp.pos = F3{__uint_as_float(C[pt]), __uint_as_float(C[64 + pt]), __uint_as_float(C[128 + pt])};
             info = C[26 * 64 + pt];
@@ -642,29 +651,36 @@ k_select(const DrJob *__restrict__ jobs, const int *list, const PointRec *pts, E
             LF[2 * LEAVES + i] = e.apmf | (pt >> 5) << 31;
             LF[3 * LEAVES + i] = (uint32_t)e.off | pt << 27;
             if (LEARNED) {
-                LF[(LW - 2) * LEAVES + i] = __float_as_uint(a.cone);
-                LF[(LW - 1) * LEAVES + i] = __float_as_uint(a.all);
+                LF[(SW - 2) * LEAVES + i] = __float_as_uint(a.cone);
+                LF[(SW - 1) * LEAVES + i] = __float_as_uint(a.all);
             }
         }
         nleaf += __popcll(m);
         if (nleaf >= 64) leaves(64);
     };
+    // entry words: TreeEntry with the point's number in the bits it leaves
+    // free (an interior node's code is below 2^30, its child offset below 2^28,
+    // a pmf's sign is unused) [, TreeAlt]
     auto pack = [&](uint32_t *x, const TreeEntry &e, TreeAlt a, uint32_t pt) {
-        x[0] = (uint32_t)e.code;
+        x[0] = (uint32_t)e.code | (pt >> 5) << 31;
         x[1] = e.cpmf;
-        x[2] = e.apmf;
-        x[3] = (uint32_t)e.off;
-        x[4] = pt;
+        x[2] = e.apmf | ((pt >> 4) & 1u) << 31;
+        x[3] = (uint32_t)e.off | pt << 28;
         if (LEARNED) {
             x[SW - 2] = __float_as_uint(a.cone);
             x[SW - 1] = __float_as_uint(a.all);
         }
     };
+    auto unpack = [&](const uint32_t *x, TreeEntry &e, TreeAlt &a) -> uint32_t {
+        e = TreeEntry{(int)(x[0] & 0x7fffffffu), x[1], x[2] & 0x7fffffffu, (int)(x[3] & 0x0fffffffu)};
+        if (LEARNED) a = TreeAlt{__uint_as_float(x[SW - 2]), __uint_as_float(x[SW - 1])};
+        return (x[0] >> 31) << 5 | (x[2] >> 31) << 4 | x[3] >> 28;
+    };
     // Fetches points until one is pending or none are left, then starts
     // pending points of one job.  False when nothing could be started now.
     auto start = [&]() -> bool {
         while (more && !__ballot(pending >= 0)) {
-            const int fetch = min(fetch_max, max(fetch_min, (int)min((float)left * share, 64.f)));
+            const int fetch = min(fetch_max, max(fetch_min, (int)min((float)left * share, 16.f)));
             unsigned long long b = 0;
             if (lane == 0) b = atomicAdd(&cnt[DR_CNT_WORK + 16 * piece], (unsigned long long)fetch);
             // the list index of the piece's f-th point (a piece: every eighth block of 256 points)
@@ -728,77 +744,74 @@ k_select(const DrJob *__restrict__ jobs, const int *list, const PointRec *pts, E
         add_leaf(lf, rs.e, rs.a, pt);
         uint32_t x[SW];
         pack(x, rs.e, rs.a, pt);
-        st.push(root && !lf, x, lane);
+        cst.push(root && !lf, x, lane);
         return true;
     };
 
-    while (true) {
-        // new points when columns are free and lanes would stay idle
-        if ((used < 32 || out0 == 0 || out1 == 0) && st.blocks == 0 && st.n + __popcll(__ballot(has)) < 64) {
-            if (start()) continue;
-        }
-        // (a stack that is almost full is worked off by lane 0 alone)
-        const bool thr = st.throttled();
-        const bool on = !thr || lane == 0;
+    // one node per lane with `on`, from the cone pass's stack or the other one
+    auto expand = [&](auto cone, WaveStack<SW> &st, bool on) {
+        constexpr bool CONE = decltype(cone)::value;
+        const DrJob &J = jobs[job];
         uint32_t x[SW];
-        if (st.pop(!has && on, x, lane)) {
-            for (int r = 0; r < SW; r++) cur[r] = x[r];
-            has = true;
-        }
-        if (!__ballot(has)) {
-            if (nleaf == 0) break;  // nothing pending, nothing to start
-            leaves(nleaf);
-            continue;
-        }
-        const bool run = has && on;
-        const uint32_t pt = cur[4];
-        TreeEntry c0, c1;
-        TreeAlt a0{0.f, 0.f}, a1{0.f, 0.f};
+        const bool run = st.pop(on, x, lane);
+        TreeEntry e{}, c0{}, c1{};
+        TreeAlt ea{0.f, 0.f}, a0{0.f, 0.f}, a1{0.f, 0.f};
         bool v0 = false, v1 = false;
+        uint32_t pt = 0;
         if (run) {
-            const DrJob &J = jobs[job];
+            pt = unpack(x, e, ea);
             EdgeTraversal T;
             SPoint sp;
             load_point(pt, J, T, sp);
-            TreeEntry e{(int)cur[0], cur[1], cur[2], (int)cur[3]};
-            TreeAlt ea{0.f, 0.f};
-            if (LEARNED) ea = TreeAlt{__uint_as_float(cur[SW - 2]), __uint_as_float(cur[SW - 1])};
-            int k = et_expand(T, e, ea, J.S, sp, c0, a0, c1, a1);
+            int k = et_expand<CONE>(T, e, ea, J.S, sp, c0, a0, c1, a1);
             // children whose bound is 0 take nothing
             v0 = k > 0 && !c0.empty();
             v1 = k > 1 && !c1.empty();
-            has = false;
         }
-        {
-            const DrJob &J = jobs[job];
+        if (J.S.stats) {
             const int k = __popcll(__ballot(run));
-            if (J.S.stats && lane == 0) atomicAdd(&J.S.stats[5], (unsigned long long)k);
+            if (lane == 0) atomicAdd(&J.S.stats[5], (unsigned long long)k);
         }
         half_count(v0, pt, out0, out1);
         half_count(v1, pt, out0, out1);
-        const bool l0 = v0 && c0.nprims() > 0, l1 = v1 && c1.nprims() > 0;
-        // the left child goes on in this lane, else the right one
-        bool p0 = v0 && !l0;
-        if (v1 && !l1) {
-            pack(cur, c1, a1, pt);
-            has = true;
-        } else if (p0) {
-            pack(cur, c0, a0, pt);
-            has = true;
-            p0 = false;
-        }
-        pack(x, c0, a0, pt);
-        st.push(p0, x, lane);
         int d0 = 0, d1 = 0;
         half_count(run, pt, d0, d1);
         out0 -= d0;
         out1 -= d1;
-        add_leaf(l0, c0, a0, pt);
-        add_leaf(l1, c1, a1, pt);
-        // a half may only wait for its last leaves
-        if (nleaf >= 16 && used == 32 && out0 > 0 && out1 > 0 && st.blocks == 0 && st.n + __popcll(__ballot(has)) < 64 &&
-             (more || __ballot(pending >= 0)))
-            leaves(nleaf);
+        auto put = [&](bool v, const TreeEntry &c, TreeAlt a) {
+            const bool leaf = v && c.nprims() > 0;
+            const bool nc = CONE && et_need_cone(c, a);
+            pack(x, c, a, pt);
+            if (CONE) cst.push(v && !leaf && nc, x, lane);
+            ast.push(v && !leaf && !nc, x, lane);
+            add_leaf(leaf, c, a, pt);
+        };
+        put(v0, c0, a0);
+        put(v1, c1, a1);
+    };
+
+    while (true) {
+        const int na = ast.size(), nc = cst.size();
+        if (na < 64 && nc < 64) {
+            // new points where columns are free, so that no lanes stay idle
+            if ((used < 32 || out0 == 0 || out1 == 0) && start()) continue;
+            // (points may only wait for their last leaves)
+            if (nleaf >= 16 && (more || __ballot(pending >= 0))) {
+                leaves(nleaf);
+                continue;
+            }
+            if (na + nc == 0) {
+                if (nleaf == 0) break;  // nothing pending, nothing to start
+                leaves(nleaf);
+                continue;
+            }
+        }
+        // a stack that is almost full is worked off by lane 0 alone, first
+        // the one that expansions of either kind push to
+        const bool ta = ast.throttled(), tc = cst.throttled();
+        const bool on = !(ta || tc) || lane == 0;
+        if (ta || (!tc && (na >= 64 || (nc < 64 && na >= nc)))) expand(std::false_type(), ast, on);
+        else expand(std::true_type(), cst, on);
     }
 }
 
@@ -1287,7 +1300,7 @@ struct LaunchTimer {
 struct Tuning {
     long long pass_samples = 1ll << 22;
     long long min_threads = 1ll << 20;
-    int select_refill = 64;  // 1-64: depth first with that refill threshold; 0: breadth first
+    int select_refill = 64;  // 1-64: depth first, fetching at most that many points at a time; 0: breadth first
 };
 
 // Device working set of the pipeline, grown on demand, and the hipGraph of
@@ -2884,7 +2897,7 @@ dr_status dr_batch_autotune(dr_batch *b, const dr_job *jobs, int num_jobs, void 
             }
         }
     }
-    // then the refill threshold of the edge selection, at the chosen pass sizes
+    // then the largest fetch of the edge selection, at the chosen pass sizes
     static const int kRefill[] = {8, 16, 32, 0};
     if (has_edges(P)) {
         for (int rf : kRefill) {

@@ -479,8 +479,8 @@ class Batch:
 
     def set_tuning(self, pass_samples, min_threads, select_refill=64):
         """select_refill: 1-64 = depth-first edge selection (the default 64),
-        with the idle lanes a wave gathers before starting new shading
-        points; 0 = breadth first."""
+        with the most shading points a wave takes at a time; 0 = breadth
+        first."""
         t = _abi.dr_tuning(pass_samples, min_threads, select_refill, 0.0, 0)
         _abi.check(self.lib, self.lib.dr_batch_set_tuning(self.handle, ctypes.byref(t)), "dr_batch_set_tuning")
 
