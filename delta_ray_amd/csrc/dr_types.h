@@ -2,8 +2,9 @@
 // and the kernels (render.hip).  Plain data only.
 //
 // HBM layout (all arrays 16-byte aligned, one allocation per array):
-//   nodes      BVH2 nodes, 64 B: both child boxes in the parent so one node
-//              fetch tests two boxes (one 64 B cache-line-friendly load)
+//   nodes      BVH2 nodes, 64 B: both child boxes in the parent (refits)
+//   packed     the same nodes as ray walks read them, 32 B: both child boxes
+//              on a 16-bit grid, so one fetch of 32 B tests two boxes
 //   tris       48 B per triangle in leaf order: v0, e1 = v1-v0, e2 = v2-v0
 //              (float4 each; v0.w carries the global triangle id)
 //   verts      float3 per global vertex (all shapes concatenated)
@@ -35,6 +36,18 @@ struct DrNode {
     float a[4], b[4], c[4];
     int d[4];
 };
+
+// What ray walks read of a node: the planes of both child boxes on a 16-bit
+// grid over the root's box, rounded outward by at least one step, so that a
+// packed box holds the exact one; half the bytes of a DrNode.  w[0..5]: lo x, y,
+// z, hi x, y, z of child 0 (low half) and child 1 (high half); w[6], w[7]: the
+// children, node index or ~(2 * first triangle slot + count - 1) for a leaf
+// (the builders make leaves of one or two triangles).  The array starts with
+// the grid (DR_PACKED_HEAD elements): lo[3], scale[3], 1 / scale[3].
+struct alignas(16) DrPackedNode {
+    uint32_t w[8];
+};
+#define DR_PACKED_HEAD 2
 
 struct DrTri {
     float v0[4];  // w: global triangle id (int bits)
@@ -101,6 +114,7 @@ struct DrCamera {
 #endif
 struct DrSceneView {
     const DR_GLOBAL DrNode *nodes;
+    const DR_GLOBAL DrPackedNode *packed;
     const DR_GLOBAL DrTri *tris;
     const DR_GLOBAL float *verts;
     const DR_GLOBAL int *tri_vidx;

@@ -16,6 +16,8 @@ struct RefitView {
     DrTri *tris;
     int num_tris;
     DrNode *nodes;
+    DrPackedNode *packed;
+    int num_nodes;
     const int *bvh_lv, *bvh_lv_off;
     int bvh_nlev;
     // mesh edges kept by the filter (sorted) and all candidates with the
@@ -53,6 +55,9 @@ struct PrimaryOut {
     float *func_int;      // device: the distribution's integral
 };
 
+// the packed copy of a BVH's nodes (dr_bvh_pack.h); packed: n + DR_PACKED_HEAD
+// elements
+void pack_bvh(const DrNode *nodes, int n, DrPackedNode *packed, hipStream_t st);
 // triangle records and BVH boxes
 void refit_geometry(const RefitView &v, hipStream_t st);
 // adds to *changed (device) the candidate edges whose filter verdict changed

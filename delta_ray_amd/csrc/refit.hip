@@ -21,6 +21,8 @@
 // All of it is compiled with -ffp-contract=off, as the host builder.
 #include "refit.h"
 
+#include "dr_bvh_pack.h"
+
 #include "dr_math.h"
 
 #define RF_BLOCK 256
@@ -445,10 +447,23 @@ namespace drrefit {
 
 static unsigned grid(long long n, int b) { return (unsigned)((n + b - 1) / b); }
 
+__global__ void k_pack_bvh(const DrNode *__restrict__ nodes, int n, DrPackedNode *__restrict__ packed) {
+    int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const BvhGrid g = bvh_grid(nodes[0]);
+    if (i == 0)
+        for (int k = 0; k < DR_PACKED_HEAD; k++) packed[k] = pack_head(g, k);
+    packed[DR_PACKED_HEAD + i] = pack_node(nodes[i], g);
+}
+void pack_bvh(const DrNode *nodes, int n, DrPackedNode *packed, hipStream_t st) {
+    if (n > 0) k_pack_bvh<<<grid(n, RF_BLOCK), RF_BLOCK, 0, st>>>(nodes, n, packed);
+}
+
 void refit_geometry(const RefitView &v, hipStream_t st) {
     if (v.num_tris > 0) k_refit_tris<<<grid(v.num_tris, RF_BLOCK), RF_BLOCK, 0, st>>>(v.tris, v.verts, v.tri_vidx, v.num_tris);
     if (v.bvh_nlev > 0)
         k_refit_bvh<<<1, RF_TREE_BLOCK, 0, st>>>(v.nodes, v.tris, v.verts, v.tri_vidx, v.bvh_lv, v.bvh_lv_off, v.bvh_nlev);
+    pack_bvh(v.nodes, v.num_nodes, v.packed, st);
 }
 
 void edge_filter(const RefitView &v, unsigned int *changed, hipStream_t st) {

@@ -1514,6 +1514,15 @@ static bool upload_structures(dr_scene *s) {
     v.prim_cdf = (decltype(v.prim_cdf))st.prim_bufs[2];
     v.num_tris = (int)hs.tri_shape.size();
     v.num_nodes = (int)hs.nodes.size();
+    v.packed = nullptr;
+    if (v.num_nodes > 0) {
+        void *pn = nullptr;
+        if (!alloc_to(A, (hs.nodes.size() + DR_PACKED_HEAD) * sizeof(DrPackedNode), &pn)) return false;
+        v.packed = (decltype(v.packed))pn;
+        drrefit::pack_bvh((const DrNode *)v.nodes, v.num_nodes, (DrPackedNode *)pn, nullptr);
+        // (renders may run on streams that do not wait for this one)
+        if (hipStreamSynchronize(nullptr) != hipSuccess) return false;
+    }
     v.num_sil_nodes = (int)hs.sil_nodes.size();
     v.num_nrm_nodes = (int)hs.nrm_nodes.size();
     v.num_sil_edges = (int)hs.sil_edges.size();
@@ -2268,6 +2277,8 @@ static drrefit::RefitView refit_view(dr_scene *s) {
     r.tris = (DrTri *)(v.tris);
     r.num_tris = (int)s->hs.tris.size();
     r.nodes = (DrNode *)(v.nodes);
+    r.packed = (DrPackedNode *)(v.packed);
+    r.num_nodes = v.num_nodes;
     r.bvh_lv = st.bvh_lv;
     r.bvh_lv_off = st.bvh_lv_off;
     r.bvh_nlev = st.bvh_nlev;
