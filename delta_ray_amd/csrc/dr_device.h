@@ -230,7 +230,8 @@ DR_INLINE Isect trace_closest(const DrSceneView &S, F3 org, F3 dir, float tmin, 
 // Culling with a ray's current closest distance is conservative and the
 // closest hit does not depend on the visiting order, so each result is the
 // one trace_closest returns for that ray.  The walk is a state advanced one
-// node at a time.
+// node at a time, so that a kernel can give a lane new rays as soon as its
+// walk ends.
 struct Walk2 {
     F3 org, da, db;
     BoxRay ra, rb;

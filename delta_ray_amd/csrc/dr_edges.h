@@ -369,12 +369,17 @@ DR_INLINE void wave_lds_fence() {
     __builtin_amdgcn_wave_barrier();
 #endif
 }
+// the blocks in private memory, an object apart from the stack's other state
+// (an object with a runtime-indexed member is kept there as a whole)
+template <int WORDS>
+struct WaveSpill {
+    uint32_t w[DR_WSTACK_BLOCKS * WORDS];
+};
 template <int WORDS>
 struct WaveStack {
     DR_LDS uint32_t *w;  // [WORDS][DR_WSTACK_LDS]
     int n, base;         // entries in LDS: ring positions base .. base + n - 1
-    int blocks;          // blocks of 64 entries in `spill`
-    uint32_t spill[DR_WSTACK_BLOCKS * WORDS];
+    int blocks;          // blocks of 64 entries in the spill
     DR_INLINE void init(DR_LDS uint32_t *lds) {
         w = lds;
         n = base = blocks = 0;
@@ -382,13 +387,13 @@ struct WaveStack {
     DR_INLINE int size() const { return n + 64 * blocks; }
     DR_INLINE bool throttled() const { return size() > DR_WSTACK_CAP - 2 * 64 - 40; }
     // lanes with `have` push their entry, lower lanes below higher ones
-    DR_INLINE void push(bool have, const uint32_t *x, int lane) {
+    DR_INLINE void push(bool have, const uint32_t *x, int lane, WaveSpill<WORDS> &spill) {
         unsigned long long m = __ballot(have);
         int k = __popcll(m);
         if (k == 0) return;
         if (n + k > DR_WSTACK_LDS) {
             int i = (base + lane) & (DR_WSTACK_LDS - 1);
-            for (int r = 0; r < WORDS; r++) spill[blocks * WORDS + r] = w[r * DR_WSTACK_LDS + i];
+            for (int r = 0; r < WORDS; r++) spill.w[blocks * WORDS + r] = w[r * DR_WSTACK_LDS + i];
             blocks++;
             base = (base + 64) & (DR_WSTACK_LDS - 1);
             n -= 64;
@@ -403,14 +408,14 @@ struct WaveStack {
     }
     // lanes with `want` take entries from the top, lower lanes first; true
     // for the lanes that got one
-    DR_INLINE bool pop(bool want, uint32_t *x, int lane) {
+    DR_INLINE bool pop(bool want, uint32_t *x, int lane, WaveSpill<WORDS> &spill) {
         unsigned long long m = __ballot(want);
         int k = __popcll(m);
         if (n < k && blocks > 0) {
             blocks--;
             base = (base - 64) & (DR_WSTACK_LDS - 1);
             int i = (base + lane) & (DR_WSTACK_LDS - 1);
-            for (int r = 0; r < WORDS; r++) w[r * DR_WSTACK_LDS + i] = spill[blocks * WORDS + r];
+            for (int r = 0; r < WORDS; r++) w[r * DR_WSTACK_LDS + i] = spill.w[blocks * WORDS + r];
             n += 64;
             wave_lds_fence();
         }
@@ -735,14 +740,28 @@ DR_INLINE bool ltc_line_sample(F3 a, F3 b, float eu, LineSample &L) {
     return true;
 }
 
-DR_INLINE EdgeResult sample_shading_edge_point(const DrSceneView &S, float bsdf_component, float eu, const DrEdge &edge,
-                                               const LightSample &ls, const SecondarySample *ss, int nss, F3 wi,
-                                               const Isect &is, const SPoint &sp, F3 weight, F3 d_color,
-                                               bool direct_only, bool *defer = nullptr,
-                                               const float *geo = nullptr,
-                                               unsigned quirks = DR_QUIRK_EDGE_BSDF_SUM | DR_QUIRK_EDGE_HIT_JACOBIAN) {
-    EdgeResult R = EdgeResult{F3{0.f, 0.f, 0.f}, F3{0.f, 0.f, 0.f}, F3{0.f, 0.f, 0.f}};
-    if (!valid(is)) return R;
+// The first part of an edge sample: the drawn point on the edge and the two
+// side rays through it.
+struct EdgeLine {
+    F3 v0, v1;      // the edge
+    M3 M;           // from the lobe's space
+    F3 wt;          // the edge's direction there
+    float pl, m_pmf;
+    F3 sample_p;    // the point relative to the shading point
+    F3 sdir, rdir, ldir;
+    int mid, comp;  // material; BSDF component the sample counts (-1: all)
+};
+// the directions from the shading point pos to the point sample_p (relative to
+// it) on the edge v0-v1 and to either side of it
+DR_INLINE void edge_side_rays(F3 sample_p, F3 v0, F3 v1, F3 pos, F3 &sdir, F3 &rdir, F3 &ldir) {
+    F3 spn = normalize(cross(v0 - pos, v1 - pos));
+    float delta = 1e-3f * length(sample_p);
+    sdir = normalize(sample_p);
+    rdir = normalize(sdir + delta * spn);
+    ldir = normalize(sdir - delta * spn);
+}
+DR_INLINE bool edge_line(const DrSceneView &S, float bsdf_component, float eu, const DrEdge &edge, F3 wi, int shape,
+                         const SPoint &sp, const float *geo, unsigned quirks, EdgeLine &E) {
     F3 v0, v1;
     if (geo) {
         // an edge the tree selected at this point (a silhouette there), with
@@ -752,82 +771,107 @@ DR_INLINE EdgeResult sample_shading_edge_point(const DrSceneView &S, float bsdf_
         v0 = F3{A.x, A.y, A.z};
         v1 = F3{B.x, B.y, B.z};
     } else {
-        if (!is_silhouette(S, sp.pos, edge)) return R;
+        if (!is_silhouette(S, sp.pos, edge)) return false;
         const DrShape &es = S.shapes[edge.shape];
         v0 = vert(S, es.vert_off + edge.v0);
         v1 = vert(S, es.vert_off + edge.v1);
     }
-    if (abs_sum(v1 - v0) == 1e-10f) return R;
-    int mid = S.shapes[is.shape].mat;
+    if (abs_sum(v1 - v0) == 1e-10f) return false;
+    int mid = S.shapes[shape].mat;
     const DrMaterial &m = S.materials[mid];
     float dw = luminance(get_diffuse(S, m, sp.uv));
     float sw = luminance(get_specular(S, m, sp.uv));
     float ws = dw + sw;
-    if (ws <= 0.f) return R;
+    if (ws <= 0.f) return false;
     float dpmf = dw / ws, spmf = sw / ws;
     F3 n = sp.fr.n;
     F3 fx = normalize(wi - n * dot(wi, n));
     F3 fy = cross(n, fx);
     M3 iso = m3_rows(fx, fy, n);
     M3 M, Minv;
-    float m_pmf;
-    int comp;
     if (bsdf_component <= dpmf) {
         Minv = iso;
         M = inverse(Minv);
-        m_pmf = dpmf;
-        comp = 0;
+        E.m_pmf = dpmf;
+        E.comp = 0;
     } else {
         Minv = mul(inverse(get_ltc_matrix(S, mid, sp, wi)), iso);
         M = inverse(Minv);
-        m_pmf = spmf;
-        comp = 1;
+        E.m_pmf = spmf;
+        E.comp = 1;
     }
     // The reference weighs the whole BSDF by the chosen component's pmf
     // (delta_ray.cpp:86-101, 249, 296-330), so each component's line
     // density integrates the whole BSDF: twice the derivative when both
     // components are nonzero.  Without that quirk a sample counts only the
     // part of the BSDF of the component it was drawn from (unbiased).
-    if (quirks & DR_QUIRK_EDGE_BSDF_SUM) comp = -1;
+    if (quirks & DR_QUIRK_EDGE_BSDF_SUM) E.comp = -1;
+    F3 a = mul(Minv, v0 - sp.pos);
+    F3 b = mul(Minv, v1 - sp.pos);
+    if (a.z <= 0.f && b.z <= 0.f) return false;
+    if (a.z < 0.f) a = (a * b.z - b * a.z) / (b.z - a.z);
+    if (b.z < 0.f) b = (a * b.z - b * a.z) / (b.z - a.z);
+    LineSample L;
+    if (!ltc_line_sample(a, b, eu, L)) return false;
+    E.pl = L.pdf;
+    E.wt = L.wt;
+    E.v0 = v0;
+    E.v1 = v1;
+    E.M = M;
+    E.mid = mid;
+    E.sample_p = mul(M, L.vo + L.l * L.wt);
+    edge_side_rays(E.sample_p, v0, v1, sp.pos, E.sdir, E.rdir, E.ldir);
+    return true;
+}
+
+// Whether the hits of the two side rays make a boundary sample: exactly one
+// of them on the edge's faces, and neither on the shading point's triangle.
+// rc, lc: which one.
+DR_INLINE bool edge_connected(const DrEdge &edge, int shape, int tri, const Isect &ir, const Isect &il, bool &rc,
+                              bool &lc) {
+    rc = ir.shape == edge.shape && (ir.tri == edge.f0 || ir.tri == edge.f1);
+    lc = il.shape == edge.shape && (il.tri == edge.f0 || il.tri == edge.f1);
+    return !(rc == lc || (ir.shape == shape && ir.tri == tri) || (il.shape == shape && il.tri == tri));
+}
+
+// hits: the side rays' closest triangles (global ids, -1: none), when the
+// caller has traced them (and knows that they make a boundary sample of a
+// nonzero BSDF); NULL: traced here.
+DR_INLINE EdgeResult sample_shading_edge_point(const DrSceneView &S, float bsdf_component, float eu, const DrEdge &edge,
+                                               const LightSample &ls, const SecondarySample *ss, int nss, F3 wi,
+                                               const Isect &is, const SPoint &sp, F3 weight, F3 d_color,
+                                               bool direct_only, const int *hits = nullptr,
+                                               const float *geo = nullptr,
+                                               unsigned quirks = DR_QUIRK_EDGE_BSDF_SUM | DR_QUIRK_EDGE_HIT_JACOBIAN) {
+    EdgeResult R = EdgeResult{F3{0.f, 0.f, 0.f}, F3{0.f, 0.f, 0.f}, F3{0.f, 0.f, 0.f}};
+    if (!valid(is)) return R;
+    EdgeLine E;
+    if (!edge_line(S, bsdf_component, eu, edge, wi, is.shape, sp, geo, quirks, E)) return R;
+    const F3 v0 = E.v0, v1 = E.v1, sdir = E.sdir, sample_p = E.sample_p, wt = E.wt;
+    const M3 &M = E.M;
+    const float pl = E.pl, m_pmf = E.m_pmf;
+    const int mid = E.mid, comp = E.comp;
     // The reference's Jacobian of a side ray's hit point w.r.t. its direction
     // treats the ray as leaving the world origin (intersect_jacobian of
     // vector.h:690-716 gets the absolute hit position, delta_ray.cpp:329-331),
     // which scales it by (x . n) / ((x - p) . n); without that quirk the
     // hit is taken relative to the shading point p.
     const bool from_origin = (quirks & DR_QUIRK_EDGE_HIT_JACOBIAN) != 0;
-    F3 a = mul(Minv, v0 - sp.pos);
-    F3 b = mul(Minv, v1 - sp.pos);
-    if (a.z <= 0.f && b.z <= 0.f) return R;
-    if (a.z < 0.f) a = (a * b.z - b * a.z) / (b.z - a.z);
-    if (b.z < 0.f) b = (a * b.z - b * a.z) / (b.z - a.z);
-    LineSample L;
-    if (!ltc_line_sample(a, b, eu, L)) return R;
-    float l = L.l, pl = L.pdf;
-    F3 vo = L.vo, wt = L.wt;
-    F3 sample_p = mul(M, vo + l * wt);
-    F3 spn = normalize(cross(v0 - sp.pos, v1 - sp.pos));
-    float delta = 1e-3f * length(sample_p);
-    F3 sdir = normalize(sample_p);
-    F3 rdir = normalize(sdir + delta * spn);
-    F3 ldir = normalize(sdir - delta * spn);
     SPoint spr, spl;
     Isect ir, il;
-    intersect2(S, sp.pos, rdir, ldir, ir, spr, il, spl);
-    bool rc = ir.shape == edge.shape && (ir.tri == edge.f0 || ir.tri == edge.f1);
-    bool lc = il.shape == edge.shape && (il.tri == edge.f0 || il.tri == edge.f1);
-    if (rc == lc || (ir.shape == is.shape && ir.tri == is.tri) || (il.shape == is.shape && il.tri == is.tri))
-        return R;
+    if (hits) {
+        ir = isect_of(S, hits[0]);
+        il = isect_of(S, hits[1]);
+        if (valid(ir)) spr = surface_point(load_tri(S, ir), sp.pos, E.rdir, false);
+        if (valid(il)) spl = surface_point(load_tri(S, il), sp.pos, E.ldir, false);
+    } else {
+        intersect2(S, sp.pos, E.rdir, E.ldir, ir, spr, il, spl);
+    }
+    bool rc, lc;
+    if (!edge_connected(edge, is.shape, is.tri, ir, il, rc, lc)) return R;
     F3 eb = bsdf(S, mid, sp, wi, sdir);
     if (sum3(eb) < 1e-6f) return R;
     if (comp >= 0) eb = bsdf(S, mid, sp, wi, sdir, comp);
-    // with `defer`, a sample that passed the connectivity test stops here
-    // and is reported: the caller runs it again in full in a launch of such
-    // samples only (about one in five), so the evaluation and continuation
-    // code runs on full waves
-    if (defer) {
-        *defer = true;
-        return R;
-    }
     F3 shr = F3{0.f, 0.f, 0.f}, shl = F3{0.f, 0.f, 0.f};
     if (!direct_only) {
         shr = shade(S, -sdir, ir, spr, ls, ss, nss, false);

@@ -394,11 +394,11 @@ DR_INLINE bool select_begin(const DrSceneView &S, const SampleCtx &c, const Poin
 
 // Stage C: one selected edge (reference delta_ray.cpp:904-966).  Scatters
 // the vertex derivatives of the edge and returns dp (the Dirac derivative at
-// the shading point).
+// the shading point).  hits: sample_shading_edge_point.
 template <int MAXB>
 DR_INLINE F3 stage_edge(const DrSceneView &S, const SampleCtx &c, GradSink &G, uint64_t sid, int b,
                         const PointRec &p, const DrEdge &edge, float w, int j, F3 d_color, float *mag = nullptr,
-                        bool *defer = nullptr, const float *geo = nullptr) {
+                        const int *hits = nullptr, const float *geo = nullptr) {
     Philox prng;
     philox_init(prng, c.seed, 0, sid, dr_stream_point(b));
     float bcomp = philox_next(prng), eu = philox_next(prng);
@@ -411,8 +411,7 @@ DR_INLINE F3 stage_edge(const DrSceneView &S, const SampleCtx &c, GradSink &G, u
     F3 weight = p.thr * ((1.f / c.spp) * w);
     Isect is = Isect{p.shape, p.tri, p.gtri};
     EdgeResult er = sample_shading_edge_point(S, bcomp, eu, edge, els, ess, nss, p.wi, is, p.sp, weight, d_color,
-                                              c.nb == 1, defer, geo, c.flags);
-    if (defer && *defer) return F3{0.f, 0.f, 0.f};
+                                              c.nb == 1, hits, geo, c.flags);
     if (!is_zero(er.dv0) || !is_zero(er.dv1)) {
         const DrShape &es = S.shapes[edge.shape];
         G.add3(es.vgrad_off + 3ll * edge.v0, er.dv0);

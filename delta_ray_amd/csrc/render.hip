@@ -9,8 +9,9 @@
 //               PointRec per (sample, bounce) shading point
 //     k_sel_points, k_select  list of the shading points; edge-tree traversal
 //               of a wave's points together -> queue of edges
-//     k_edge    thread = one selected edge: secondary edge sample, vertex
-//               gradients, Dirac position derivative dp of its point
+//     k_edge_draw, k_edge_trace, k_edge_shade  thread = one selected edge:
+//               secondary edge sample, its side rays, then vertex gradients
+//               and the Dirac position derivative dp of its point
 //     k_dp_last keeps the last dp per point (set_adjoint overwrite)
 //     k_dp      replays the path to propagate dp (2nd adjoint sweep)
 //   k_primary   primary-edge samples (reference pass 2, delta_ray.cpp:1468-1550)
@@ -79,10 +80,6 @@ DR_INLINE int range_of_block(const DrRange *r, int n, long long b) {
 
 #define DR_GC_SLOTS_BIG 4096
 #define DR_GC_SLOTS_SMALL 2048
-// k_edge: 1024 slots (12 KB) + the ray stack (16 KB) leave room for five
-// workgroups per CU, which its 96-VGPR budget also allows (5 % faster than
-// 2048 slots at four)
-#define DR_GC_SLOTS_EDGE 1024
 
 // thread -> (pixel, chunk of `per` samples) of a forward-only job
 __global__ void __launch_bounds__(DR_BLOCK) k_forward(const DrJob *__restrict__ jobs, const DrRange *__restrict__ R,
@@ -111,10 +108,15 @@ __global__ void __launch_bounds__(DR_BLOCK) k_forward(const DrJob *__restrict__ 
 // slot0 + ((t - t0) * per + k) * MAXB + b.
 struct EdgeEntry {
     int slot;  // point slot in the pass
-    int edge;  // index into the tree's edge list; bit 31 set: normal tree
+    int edge;  // index into the tree's edge list; bit 31 set: normal tree; bit 30: selected by the "all" pass
     float w;
-    int j;     // ordinal of the edge in its pass (bit 30: the "all" pass)
+    int list;  // k_edge_draw: an element of the list of drawn samples, unrelated to this entry
+    DR_INLINE int index() const { return edge & 0x07ffffff; }
+    DR_INLINE bool normal() const { return (edge & 0x80000000) != 0; }
+    // the edge's ordinal in its pass (bit 30: the "all" pass)
+    DR_INLINE int ordinal() const { return edge & (DR_ORD_ALL_PASS | 0x07ffffff); }
 };
+static_assert(DR_ORD_ALL_PASS == 0x40000000 && DR_EDGE_ORDINAL_BITS == 27, "EdgeEntry.edge holds the ordinal");
 
 
 template <int MAXB>
@@ -406,7 +408,7 @@ __global__ void __launch_bounds__(DR_BLOCK) k_sel_leaves(const DrJob *__restrict
                 auto emit = [&](float w, bool nrm, int idx, int ord) {
                     calls++;
                     if (w != 0.f) {
-                        EdgeEntry y{E.slot, idx | (nrm ? (int)0x80000000 : 0), w, ord};
+                        EdgeEntry y{E.slot, ord | (nrm ? (int)0x80000000 : 0), w, 0};
                         if (got == 0) y0 = y;
                         else y1 = y;
                         got++;
@@ -437,7 +439,9 @@ __global__ void __launch_bounds__(DR_BLOCK) k_sel_leaves(const DrJob *__restrict
 // clears the slots' edge counts.
 #define DR_CNT_POINTS 6                        // word of the counters: points listed
 #define DR_CNT_WORK 16                         // first of the list's eight work counters, 16 words apart
-#define DR_CNT_WORDS (DR_CNT_WORK + 8 * 16)
+#define DR_CNT_DRAWN (DR_CNT_WORK + 8 * 16)    // edge samples drawn (k_edge_draw)
+#define DR_CNT_CLAIM (DR_CNT_DRAWN + 16)       // first of their eight work counters, 16 words apart
+#define DR_CNT_WORDS (DR_CNT_CLAIM + 8 * 16)
 #define DR_LIST_PER_THREAD 8
 __global__ void __launch_bounds__(DR_BLOCK) k_sel_points(long long nslots, int maxb, const PointRec *pts, int *list,
                                                          unsigned long long *cnt, int *counts, long long f_begin,
@@ -526,6 +530,7 @@ k_select(const DrJob *__restrict__ jobs, const int *list, const PointRec *pts, E
     const long long npoints = (long long)cnt[DR_CNT_POINTS];
     const int lane = (int)__lane_id();
     WaveStack<SW> cst, ast;  // nodes with and without et_need_cone
+    WaveSpill<SW> cspill, aspill;
     cst.init((DR_LDS uint32_t *)s_stack[0]);
     ast.init((DR_LDS uint32_t *)s_stack[1]);
     int nleaf = 0, leaf0 = 0;  // leaves waiting (a ring), the oldest
@@ -609,7 +614,7 @@ k_select(const DrJob *__restrict__ jobs, const int *list, const PointRec *pts, E
                     calls++;
                     // zero-weight edges carry no work (reference delta_ray.cpp:906-908)
                     if (w != 0.f) {
-                        EdgeEntry y{slot, idx | (nrm ? (int)0x80000000 : 0), w, ord};
+                        EdgeEntry y{slot, ord | (nrm ? (int)0x80000000 : 0), w, 0};
                         if (ke == 0) y0 = y;
                         else y1 = y;
                         ke++;
@@ -682,9 +687,13 @@ k_select(const DrJob *__restrict__ jobs, const int *list, const PointRec *pts, E
         while (more && !__ballot(pending >= 0)) {
             const int fetch = min(fetch_max, max(fetch_min, (int)min((float)left * share, 16.f)));
             unsigned long long b = 0;
-            if (lane == 0) b = atomicAdd(&cnt[DR_CNT_WORK + 16 * piece], (unsigned long long)fetch);
             // the list index of the piece's f-th point (a piece: every eighth block of 256 points)
             auto at = [&](long long f) { return ((f >> 8) * 8 + piece) * 256 + (f & 255); };
+            // (at the others' pieces a plain look first: most are used up)
+            if (lane == 0) {
+                if (tried > 0) b = __atomic_load_n(&cnt[DR_CNT_WORK + 16 * piece], __ATOMIC_RELAXED);
+                if (at((long long)b) < npoints) b = atomicAdd(&cnt[DR_CNT_WORK + 16 * piece], (unsigned long long)fetch);
+            }
             const long long f = (long long)__shfl(b, 0);
             const long long i = at(f + lane);
             if (lane < fetch && i < npoints) pending = list[i];
@@ -744,16 +753,16 @@ k_select(const DrJob *__restrict__ jobs, const int *list, const PointRec *pts, E
         add_leaf(lf, rs.e, rs.a, pt);
         uint32_t x[SW];
         pack(x, rs.e, rs.a, pt);
-        cst.push(root && !lf, x, lane);
+        cst.push(root && !lf, x, lane, cspill);
         return true;
     };
 
     // one node per lane with `on`, from the cone pass's stack or the other one
-    auto expand = [&](auto cone, WaveStack<SW> &st, bool on) {
+    auto expand = [&](auto cone, WaveStack<SW> &st, WaveSpill<SW> &spill, bool on) {
         constexpr bool CONE = decltype(cone)::value;
         const DrJob &J = jobs[job];
         uint32_t x[SW];
-        const bool run = st.pop(on, x, lane);
+        const bool run = st.pop(on, x, lane, spill);
         TreeEntry e{}, c0{}, c1{};
         TreeAlt ea{0.f, 0.f}, a0{0.f, 0.f}, a1{0.f, 0.f};
         bool v0 = false, v1 = false;
@@ -782,8 +791,8 @@ k_select(const DrJob *__restrict__ jobs, const int *list, const PointRec *pts, E
             const bool leaf = v && c.nprims() > 0;
             const bool nc = CONE && et_need_cone(c, a);
             pack(x, c, a, pt);
-            if (CONE) cst.push(v && !leaf && nc, x, lane);
-            ast.push(v && !leaf && !nc, x, lane);
+            if (CONE) cst.push(v && !leaf && nc, x, lane, cspill);
+            ast.push(v && !leaf && !nc, x, lane, aspill);
             add_leaf(leaf, c, a, pt);
         };
         put(v0, c0, a0);
@@ -810,29 +819,254 @@ k_select(const DrJob *__restrict__ jobs, const int *list, const PointRec *pts, E
         // the one that expansions of either kind push to
         const bool ta = ast.throttled(), tc = cst.throttled();
         const bool on = !(ta || tc) || lane == 0;
-        if (ta || (!tc && (na >= 64 || (nc < 64 && na >= nc)))) expand(std::false_type(), ast, on);
-        else expand(std::true_type(), cst, on);
+        if (ta || (!tc && (na >= 64 || (nc < 64 && na >= nc)))) expand(std::false_type(), ast, aspill, on);
+        else expand(std::true_type(), cst, cspill, on);
     }
 }
 
-// C: one selected edge per iteration of a grid-stride loop over the queue
-// (its length is read on the device, so no host round trip is needed).  Only
-// about one edge sample in five passes the connectivity test of its two side
-// rays (the rest stop at the horizon, at that test or at a zero BSDF), and
-// what follows (evaluation at both hits, continuation paths, the Dirac
-// Jacobians, the scatter) is the longest code of the kernel: run in the same
-// waves it would leave most lanes idle.  So k_edge stops such samples there
-// (returns true: nothing of theirs is written) and appends them to a list;
-// k_edge_shade then runs them in full, on full waves.  Every sample is thus
-// computed by exactly one launch, with the same operations as in one pass.
+// C: edge samples.  Only about one in five passes the connectivity test of its
+// two side rays (the rest stop at the horizon, at a zero BSDF or at that test), and what
+// follows (evaluation at both hits, continuation paths, the Dirac Jacobians,
+// the scatter) is long code.  So the samples go through three kernels:
+//   k_edge_draw   draws every sample's point on its edge and lists the samples
+//                 that have one with a nonzero BSDF (about half);
+//   k_edge_trace  walks their side rays and lists the samples that pass, with
+//                 the rays' triangles;
+//   k_edge_shade  runs those in full, on full waves.
+// Walking the rays is a chain of node loads, bound by their latency and by
+// the divergence of the walks' lengths, so it has a kernel of its own, whose
+// few registers leave room for five waves per SIMD and where a lane takes a new
+// sample when its walk ends.  What it needs of a sample is its point on the
+// edge (in entry_dp, which is written at the end only) and what the queue entry
+// refers to.  On the heightfield (182 M samples a render of four passes) the
+// three take 3.2 + 8.5 + 6.5 ms a pass; drawing and walking in one kernel, one
+// sample a thread, and the walks again before the evaluation 20.7 + 12.7 (on
+// 64-byte nodes).
+//
+// The length of the queue is read on the device, so no host round trip is
+// needed.  cnt[2] keeps the largest queue length seen, for the host's overflow
+// check; cnt[3] counts the samples for k_edge_shade (listed in `cont`, which has
+// the queue's capacity; their entry_dp holds the side rays' triangles until
+// then); cnt[DR_CNT_DRAWN] the samples drawn (listed in the queue's `list`
+// words).
+DR_INLINE const DrEdge &entry_edge(const DrJob &J, const EdgeEntry &E, const float *&geo) {
+    // the edge was selected at this point, so it is a silhouette there: its
+    // endpoints come from the tree's geometry record
+    geo = (E.normal() ? J.S.nrm_geo : J.S.sil_geo) + 16 * (size_t)E.index();
+    return E.normal() ? J.S.nrm_edges[E.index()] : J.S.sil_edges[E.index()];
+}
+// the sample's edge statistics: |contribution| mag
+DR_INLINE void edge_stats(const DrJob &J, const EdgeEntry &E, float mag) {
+    if (!((J.c.flags & DR_EDGE_STATS) && J.S.edge_stat)) return;
+    long long ge = (E.normal() ? (long long)J.S.num_sil_edges : 0ll) + E.index();
+    if (mag != 0.f) {
+        atomicAdd(J.S.edge_stat + 3 * ge, mag);
+        atomicAdd(J.S.edge_stat + 3 * ge + 2, mag * mag);
+    }
+    atomicAdd(J.S.edge_stat + 3 * ge + 1, 1.f);
+}
+
+// a sample that contributes nothing: it takes no part in the last-dp rule
+DR_INLINE void edge_drop(const DrJob &J, const EdgeEntry &E, float4 *dp) {
+    edge_stats(J, E, 0.f);
+    *dp = make_float4(0.f, 0.f, 0.f, __int_as_float(-1));
+}
+
+// One sample per thread; a workgroup lists the samples of four rounds with one
+// atomic.
+#define DR_DRAW_PER_THREAD 4
+__global__ void __launch_bounds__(DR_BLOCK) k_edge_draw(const DrJob *__restrict__ jobs, EdgeEntry *q,
+                                                        unsigned long long *cnt, long long cap, const PointRec *pts,
+                                                        float4 *entry_dp) {
+    __shared__ int s_n[DR_DRAW_PER_THREAD * (DR_BLOCK / 64)];
+    __shared__ unsigned long long s_base;
+    const unsigned long long len = cnt[0];
+    if (blockIdx.x == 0 && threadIdx.x == 0) atomicMax(&cnt[2], len);
+    const long long n = (long long)len < cap ? (long long)len : cap;
+    const int lane = (int)__lane_id(), w = threadIdx.x >> 6;
+    const long long per = (long long)DR_BLOCK * DR_DRAW_PER_THREAD;
+    for (long long e0 = blockIdx.x * per; e0 < n; e0 += gridDim.x * per) {
+        int rank[DR_DRAW_PER_THREAD];
+        bool drawn[DR_DRAW_PER_THREAD];
+#pragma unroll 1
+        for (int i = 0; i < DR_DRAW_PER_THREAD; i++) {
+            const long long e = e0 + i * DR_BLOCK + threadIdx.x;
+            bool ok = false;
+            if (e < n) {
+                const EdgeEntry E = q[e];
+                const PointRec &p = pts[E.slot];
+                const DrJob &J = jobs[p.job];
+                const float *geo;
+                const DrEdge &edge = entry_edge(J, E, geo);
+                Philox prng;
+                philox_init(prng, J.c.seed, 0, p.sid, dr_stream_point(p.b));
+                const float bcomp = philox_next(prng), eu = philox_next(prng);
+                EdgeLine L;
+                ok = p.gtri >= 0 && edge_line(J.S, bcomp, eu, edge, p.wi, p.shape, p.sp, geo, J.c.flags, L) &&
+                     !(sum3(bsdf(J.S, L.mid, p.sp, p.wi, L.sdir)) < 1e-6f);
+                if (ok) entry_dp[e] = make_float4(L.sample_p.x, L.sample_p.y, L.sample_p.z, 0.f);
+                else edge_drop(J, E, entry_dp + e);
+            }
+            const unsigned long long m = __ballot(ok);
+            const int r = __popcll(m & ((1ull << lane) - 1ull));
+#pragma unroll
+            for (int k = 0; k < DR_DRAW_PER_THREAD; k++)
+                if (k == i) {
+                    drawn[k] = ok;
+                    rank[k] = r;
+                }
+            if (lane == 0) s_n[i * (DR_BLOCK / 64) + w] = __popcll(m);
+        }
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            int t = 0;
+            for (int i = 0; i < DR_DRAW_PER_THREAD * (DR_BLOCK / 64); i++) {
+                int k = s_n[i];
+                s_n[i] = t;
+                t += k;
+            }
+            s_base = t > 0 ? atomicAdd(&cnt[DR_CNT_DRAWN], (unsigned long long)t) : 0ull;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < DR_DRAW_PER_THREAD; i++)
+            if (drawn[i]) q[s_base + s_n[i * (DR_BLOCK / 64) + w] + rank[i]].list = (int)(e0 + i * DR_BLOCK + threadIdx.x);
+        __syncthreads();
+    }
+}
+
+// The drawn samples' side rays.  Walk lengths vary widely, so a lane that is
+// done waits only until DR_EDGE_REFILL lanes are: then the finished samples are
+// tested and the idle lanes take new ones together.  The list is worked off in
+// eight contiguous pieces, a workgroup beginning with its chiplet's (workgroups
+// are handed to the eight in turn): a piece's rays begin in one band of the
+// image, and each chiplet has its own L2.  A wave claims 64 to 512 samples
+// of a piece at a time (a quarter of an even share of what is left; the first
+// of every wave's claims has a fixed place, so that a short list needs no
+// atomics), and goes on with the next piece when one is used up.  One counter
+// for all and a list append of 64 samples at a time cost 1.7 ms where this
+// takes 0.6 (6 M short walks); a refill at 8 / 16 / 32 idle lanes measured
+// 10.4 / 8.8 / 8.0 ms on the heightfield (48: 3 % less than 32), four / five / six
+// waves per SIMD 9.6 / 8.8 / 9.7.
+#define DR_EDGE_REFILL 48
+#define DR_EDGE_FOUND 256
+__global__ void __launch_bounds__(DR_BLOCK) __attribute__((amdgpu_waves_per_eu(5)))
+k_edge_trace(const DrJob *__restrict__ jobs, const EdgeEntry *q, unsigned long long *cnt, const PointRec *pts,
+             float4 *entry_dp, int *cont) {
+    __shared__ int s_found[DR_BLOCK / 64][DR_EDGE_FOUND];  // per wave: samples that passed, not listed yet
+    const long long n = (long long)cnt[DR_CNT_DRAWN];
+    const int lane = (int)__lane_id();
+    DR_LDS int *found = (DR_LDS int *)s_found[threadIdx.x >> 6];
+    int nfound = 0;
+    const float share = 2.f / (float)((long long)gridDim.x * (DR_BLOCK / 64));
+    const long long psize = ((n + 7) / 8 + 63) & ~63ll;  // samples of a piece
+    auto claim = [&](long long left) { return max(64ll, min(512ll, (long long)((float)left * share))); };
+    const long long fixed = claim(psize);
+    int piece = (int)(blockIdx.x & 7), tried = 0;
+    // this wave's claim
+    const long long mine = ((long long)(blockIdx.x >> 3) * (DR_BLOCK / 64) + (threadIdx.x >> 6)) * fixed;
+    long long next = piece * psize + mine, end = min(next + fixed, min((piece + 1) * psize, n));
+    bool more = true;   // pieces may have samples left
+    int e = -1;         // this lane's sample
+    bool busy = false;  // its walk goes on
+    Walk2 w;
+    TraceStack stack;
+    // the samples found go to the list
+    auto list = [&]() {
+        wave_lds_fence();
+        unsigned long long base = 0;
+        if (lane == 0) base = atomicAdd(&cnt[3], (unsigned long long)nfound);
+        base = __shfl(base, 0);
+        for (int i = lane; i < nfound; i += 64) cont[base + i] = found[i];
+        wave_lds_fence();
+        nfound = 0;
+    };
+    while (true) {
+        // finished samples
+        bool pass = false;
+        if (e >= 0 && !busy) {
+            const EdgeEntry E = q[e];
+            const PointRec &p = pts[E.slot];
+            const DrJob &J = jobs[p.job];
+            const float *geo;
+            const DrEdge &edge = entry_edge(J, E, geo);
+            w.count(J.S);
+            bool rc, lc;
+            pass = edge_connected(edge, p.shape, p.tri, isect_of(J.S, w.ga), isect_of(J.S, w.gb), rc, lc);
+            if (pass) entry_dp[e] = make_float4(__int_as_float(w.ga), __int_as_float(w.gb), 0.f, 0.f);
+            else edge_drop(J, E, entry_dp + e);
+        }
+        unsigned long long m = __ballot(pass);
+        if (pass) found[nfound + __popcll(m & ((1ull << lane) - 1ull))] = e;
+        nfound += __popcll(m);
+        if (nfound > DR_EDGE_FOUND - 64) list();
+        if (!busy) e = -1;
+        // new samples for the idle lanes
+        while (next >= end && more) {
+            const long long first = piece * psize, size = min(psize, n - first);
+            const long long base = (long long)((gridDim.x - piece + 7) >> 3) * (DR_BLOCK / 64) * fixed;
+            // (at the others' pieces a plain look first: most are used up)
+            unsigned long long *const at = &cnt[DR_CNT_CLAIM + 16 * piece];
+            unsigned long long old = 0;
+            if (lane == 0 && tried > 0 && base < size) old = __atomic_load_n(at, __ATOMIC_RELAXED);
+            long long c = base + (long long)__shfl(old, 0);
+            const long long want = claim(size - c);
+            if (c < size) {
+                if (lane == 0) old = atomicAdd(at, (unsigned long long)want);
+                c = base + (long long)__shfl(old, 0);
+                next = first + c;
+                end = first + min(c + want, size);
+            }
+            if (c + want >= size) {
+                piece = (piece + 1) & 7;
+                if (++tried == 8) more = false;
+            }
+        }
+        m = __ballot(!busy);
+        const long long i = next + __popcll(m & ((1ull << lane) - 1ull));
+        if (next < end) next += __popcll(m);
+        if (!busy && i < end) {
+            e = q[i].list;
+            const EdgeEntry E = q[e];
+            const float4 sp = entry_dp[e];
+            const PointRec &p = pts[E.slot];
+            const DrJob &J = jobs[p.job];
+            const float *geo;
+            entry_edge(J, E, geo);
+            const DR_GLOBAL float4 *g = (const DR_GLOBAL float4 *)geo;
+            const float4 A = g[0], B = g[1];
+            F3 sdir, rdir, ldir;
+            edge_side_rays(F3{sp.x, sp.y, sp.z}, F3{A.x, A.y, A.z}, F3{B.x, B.y, B.z}, p.sp.pos, sdir, rdir, ldir);
+            busy = w.begin(J.S, p.sp.pos, rdir, ldir);
+        }
+        const bool unstarted = next < end || more;
+        if (!__ballot(busy)) {
+            if (!unstarted && !__ballot(e >= 0)) break;
+            continue;
+        }
+        // walk until enough lanes are idle, or to the end when no samples are left
+        const int stay = unstarted ? 64 - DR_EDGE_REFILL : 0;
+        const DrSceneView &J = jobs[e >= 0 ? pts[q[e].slot].job : 0].S;
+        DrSceneView S;  // (what a step reads, in registers)
+        S.packed = J.packed;
+        S.tris = J.tris;
+        S.num_nodes = J.num_nodes;
+        S.stats = J.stats;
+        do {
+            if (busy) busy = w.step(S, stack);
+        } while (__popcll(__ballot(busy)) > stay);
+    }
+    if (nfound > 0) list();
+}
+
+// The samples that passed: evaluation and continuation paths.
 template <int MAXB>
-DR_INLINE bool edge_entry(const DrJob *jobs, const EdgeEntry &E, long long e,
-                          const PointRec *pts, float *pt_dp, int *pt_lastj, float4 *entry_dp,
-                          unsigned long long *gkey, float *gval, int gslots, bool defer) {
+DR_INLINE void edge_entry(const DrJob *jobs, const EdgeEntry &E, long long e, const PointRec *pts, float *pt_dp,
+                          int *pt_lastj, float4 *entry_dp, unsigned long long *gkey, float *gval, int gslots) {
     const PointRec &p = pts[E.slot];
     const DrJob &J = jobs[p.job];
-    int idx = E.edge & 0x7fffffff;
-    const DrEdge &edge = (E.edge & 0x80000000) ? J.S.nrm_edges[idx] : J.S.sil_edges[idx];
+    const float *geo;
+    const DrEdge &edge = entry_edge(J, E, geo);
     GradSink G;
     G.grads = J.grads;
     G.cam = nullptr;
@@ -844,25 +1078,14 @@ DR_INLINE bool edge_entry(const DrJob *jobs, const EdgeEntry &E, long long e,
     G.job = (unsigned)p.job;
     F3 d_color = load3(J.d_image + 3 * (size_t)p.pix);
     float mag = 0.f;
-    bool deferred = false;
-    // the edge was selected at this point, so it is a silhouette there: its
-    // endpoints come from the tree's geometry record
-    const float *geo = ((E.edge & 0x80000000) ? J.S.nrm_geo : J.S.sil_geo) + 16 * (size_t)idx;
-    F3 dp = stage_edge<MAXB>(J.S, J.c, G, p.sid, p.b, p, edge, E.w, E.j, d_color, &mag,
-                             defer ? &deferred : nullptr, geo);
-    if (deferred) return true;
-    if ((J.c.flags & DR_EDGE_STATS) && J.S.edge_stat) {
-        long long ge = (E.edge & 0x80000000) ? (long long)J.S.num_sil_edges + idx : (long long)idx;
-        if (mag != 0.f) {
-            atomicAdd(J.S.edge_stat + 3 * ge, mag);
-            atomicAdd(J.S.edge_stat + 3 * ge + 2, mag * mag);
-        }
-        atomicAdd(J.S.edge_stat + 3 * ge + 1, 1.f);
-    }
+    const float4 h = entry_dp[e];
+    const int hits[2] = {__float_as_int(h.x), __float_as_int(h.y)};
+    F3 dp = stage_edge<MAXB>(J.S, J.c, G, p.sid, p.b, p, edge, E.w, E.ordinal(), d_color, &mag, hits, geo);
+    edge_stats(J, E, mag);
     bool nz = !is_zero(dp);
     if (J.c.flags & DR_QUIRK_DP_LAST) {
-        entry_dp[e] = make_float4(dp.x, dp.y, dp.z, nz ? __int_as_float(E.j) : __int_as_float(-1));
-        if (nz) atomicMax(pt_lastj + E.slot, E.j);
+        entry_dp[e] = make_float4(dp.x, dp.y, dp.z, nz ? __int_as_float(E.ordinal()) : __int_as_float(-1));
+        if (nz) atomicMax(pt_lastj + E.slot, E.ordinal());
     } else {
         // a pass may mix jobs with and without the last-dp rule: mark the
         // entry as not taking part in it
@@ -873,45 +1096,7 @@ DR_INLINE bool edge_entry(const DrJob *jobs, const EdgeEntry &E, long long e,
             atomicAdd(pt_dp + 3ll * E.slot + 2, dp.z);
         }
     }
-    return false;
 }
-
-// cnt[2] keeps the largest queue length seen, for the host's overflow check;
-// cnt[3] counts the samples left for k_edge_shade (listed in `cont`, which
-// has the queue's capacity).
-template <int MAXB>
-__global__ void __launch_bounds__(DR_BLOCK) __attribute__((amdgpu_waves_per_eu(5)))
-k_edge(const DrJob *__restrict__ jobs, const EdgeEntry *q, unsigned long long *cnt, long long cap,
-       const PointRec *pts, float *pt_dp, int *pt_lastj, float4 *entry_dp, int *cont) {
-    __shared__ unsigned long long gkey[DR_GC_SLOTS_EDGE];
-    __shared__ float gval[DR_GC_SLOTS_EDGE];
-    gc_init(gkey, gval, DR_GC_SLOTS_EDGE);
-    __syncthreads();
-    unsigned long long len = cnt[0];
-    if (blockIdx.x == 0 && threadIdx.x == 0) atomicMax(&cnt[2], len);
-    long long n = (long long)len < cap ? (long long)len : cap;
-    long long stride = (long long)gridDim.x * blockDim.x;
-    const int lane = (int)__lane_id();
-    for (long long e0 = (long long)blockIdx.x * blockDim.x + (threadIdx.x - lane); e0 < n; e0 += stride) {
-        // whole waves iterate together (e0: the wave's first entry), so the
-        // list append below is one atomic per wave
-        long long e = e0 + lane;
-        bool later = e < n && edge_entry<MAXB>(jobs, q[e], e, pts, pt_dp, pt_lastj, entry_dp, gkey, gval,
-                                               DR_GC_SLOTS_EDGE, true);
-        unsigned long long m = __ballot(later);
-        if (m) {
-            int leader = __ffsll((long long)m) - 1;
-            unsigned long long base = 0;
-            if (lane == leader) base = atomicAdd(&cnt[3], (unsigned long long)__popcll(m));
-            base = __shfl(base, leader);
-            if (later) cont[base + __popcll(m & ((1ull << lane) - 1ull))] = (int)e;
-        }
-    }
-    __syncthreads();
-    gc_flush(gkey, gval, DR_GC_SLOTS_EDGE, [&](int j) { return jobs[j].grads; });
-}
-
-// C': the samples k_edge left for the continuation paths, in full.
 template <int MAXB>
 __global__ void __launch_bounds__(DR_BLOCK) __attribute__((amdgpu_waves_per_eu(2)))
 k_edge_shade(const DrJob *__restrict__ jobs, const EdgeEntry *q,
@@ -926,7 +1111,7 @@ k_edge_shade(const DrJob *__restrict__ jobs, const EdgeEntry *q,
     long long stride = (long long)gridDim.x * blockDim.x;
     for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
         long long e = cont[i];
-        edge_entry<MAXB>(jobs, q[e], e, pts, pt_dp, pt_lastj, entry_dp, gkey, gval, DR_GC_SLOTS_BIG, false);
+        edge_entry<MAXB>(jobs, q[e], e, pts, pt_dp, pt_lastj, entry_dp, gkey, gval, DR_GC_SLOTS_BIG);
     }
     __syncthreads();
     gc_flush(gkey, gval, DR_GC_SLOTS_BIG, [&](int j) { return jobs[j].grads; });
@@ -1106,6 +1291,7 @@ DR_INLINE void tree_stack_run(long long ops, uint64_t seed, DR_LDS uint32_t *lds
     const int lane = (int)__lane_id();
     const uint64_t wave = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
     WaveStack<WORDS> A;
+    WaveSpill<WORDS> spill;
     A.init(lds);
     uint32_t ref[32];  // the operation that pushed the entry
     int size = 0, deepest = 0;
@@ -1126,7 +1312,7 @@ DR_INLINE void tree_stack_run(long long ops, uint64_t seed, DR_LDS uint32_t *lds
             mine = mine && size + rank < DR_WSTACK_CAP;
             int n = __popcll(__ballot(mine));
             for (int r = 0; r < WORDS; r++) x[r] = word(size + rank, (uint32_t)k, r);
-            A.push(mine, x, lane);
+            A.push(mine, x, lane, spill);
             for (int i = 0; i < 32; i++) {
                 int p = i * 64 + lane;
                 if (p >= size && p < size + n) ref[i] = (uint32_t)k;
@@ -1135,7 +1321,7 @@ DR_INLINE void tree_stack_run(long long ops, uint64_t seed, DR_LDS uint32_t *lds
         } else {
             unsigned long long m = __ballot(mine);
             int rank = __popcll(m & ((1ull << lane) - 1ull));
-            bool got = A.pop(mine, x, lane);
+            bool got = A.pop(mine, x, lane, spill);
             int n = __popcll(__ballot(got));
             // the plain array's entry at position size - 1 - rank: lanes get
             // min(asked, stack) entries whenever the ring and one block hold
@@ -1313,14 +1499,15 @@ struct Workspace {
     long long slot_cap = 0;
     EdgeEntry *q = nullptr;
     float4 *entry_dp = nullptr;
-    // queue entries left for the continuation launch (k_edge), and before it
+    // queue entries left for k_edge_shade, and before them
     // the list of the pass's points (k_sel_points: at most one per slot, and
     // the queue has at least an entry per slot)
     int *cont = nullptr;
     long long q_cap = 0;
-    // queue length, unused, largest queue length, continuations, largest
-    // frontier end, largest leaf-list end (breadth-first selection), points
-    // listed (DR_CNT_POINTS), unused; then the list's work counters
+    // queue length, -, largest queue length, continuations, largest frontier
+    // end, largest leaf-list end (breadth-first selection), points listed
+    // (DR_CNT_POINTS); then the point list's work counters, the samples drawn
+    // and their work counters
     unsigned long long *cnt = nullptr;
     unsigned long long *cnt_host = nullptr;  // pinned, 8 words
     SelPoint *spt = nullptr;                 // breadth-first selection: per point slot
@@ -1862,7 +2049,7 @@ static dr_status grow_queue(Workspace &w, long long n) {
     return DR_OK;
 }
 
-static long long g_select_blocks[2] = {0, 0}, g_edge_blocks[4] = {0, 0, 0, 0}, g_shade_blocks[4] = {0, 0, 0, 0};
+static long long g_select_blocks[2] = {0, 0}, g_trace_blocks = 0, g_draw_blocks = 0, g_shade_blocks[4] = {0, 0, 0, 0};
 static long long g_sel_blocks[3] = {0, 0, 0};
 
 // All launches of a plan, stream-ordered, without host synchronisation (so
@@ -1915,13 +2102,23 @@ static void launch_select(const Plan &P, const Workspace &w, long long nslots, i
     int fetch_min = std::min(fetch_max, std::max(4, std::min(64, 4096 / std::max(1, P.tree_nodes))));
     unsigned grid = (unsigned)std::min<long long>(waves, (n + fetch_min - 1) / fetch_min);
     const int per_block = DR_BLOCK * DR_LIST_PER_THREAD;
-    k_fill<<<1, 256, 0, hs>>>((float *)(w.cnt + DR_CNT_POINTS), 2 * (DR_CNT_WORDS - DR_CNT_POINTS), 0.f);
+    k_fill<<<1, 256, 0, hs>>>((float *)(w.cnt + DR_CNT_POINTS), 2 * (DR_CNT_DRAWN - DR_CNT_POINTS), 0.f);
     k_sel_points<<<(unsigned)((n + per_block - 1) / per_block), DR_BLOCK, 0, hs>>>(nslots, maxb, w.pts, w.cont, w.cnt,
                                                                                   w.counts, f0, f1);
     if (P.learned)
         k_select<true><<<grid, 64, 0, hs>>>(w.jobs, w.cont, w.pts, w.q, w.cnt, w.q_cap, w.counts, fetch_min, fetch_max);
     else
         k_select<false><<<grid, 64, 0, hs>>>(w.jobs, w.cont, w.pts, w.q, w.cnt, w.q_cap, w.counts, fetch_min, fetch_max);
+}
+
+// The selected edges' samples up to their side rays (resident grids: the
+// queue's length is known on the device only).
+static void launch_edge_trace(const Workspace &w, hipStream_t hs) {
+    k_fill<<<1, 256, 0, hs>>>((float *)(w.cnt + DR_CNT_DRAWN), 2 * (DR_CNT_WORDS - DR_CNT_DRAWN), 0.f);
+    k_edge_draw<<<(unsigned)resident_blocks(k_edge_draw, g_draw_blocks), DR_BLOCK, 0, hs>>>(w.jobs, w.q, w.cnt, w.q_cap,
+                                                                                           w.pts, w.entry_dp);
+    k_edge_trace<<<(unsigned)resident_blocks(k_edge_trace, g_trace_blocks), DR_BLOCK, 0, hs>>>(w.jobs, w.q, w.cnt, w.pts,
+                                                                                              w.entry_dp, w.cont);
 }
 
 template <class Launch>
@@ -1986,11 +2183,9 @@ static dr_status enqueue(const Plan &P, Workspace &w, Timing *tm, hipStream_t hs
             dr_status st = settle_selection(w, hs, bfs, select);
             if (st != DR_OK) return st;
         }
-        long long eb = resident_blocks(k_edge<MAXB>, g_edge_blocks[bi]);
         {
             LaunchTimer t(tm, TK_EDGE, hs);
-            k_edge<MAXB><<<(unsigned)eb, DR_BLOCK, 0, hs>>>(w.jobs, w.q, w.cnt, w.q_cap, w.pts, w.pt_dp, w.pt_lastj,
-                                                            w.entry_dp, w.cont);
+            launch_edge_trace(w, hs);
         }
         {
             LaunchTimer t(tm, TK_SHADE, hs);
@@ -1998,7 +2193,7 @@ static dr_status enqueue(const Plan &P, Workspace &w, Timing *tm, hipStream_t hs
             k_edge_shade<MAXB><<<(unsigned)sb, DR_BLOCK, 0, hs>>>(w.jobs, w.q, w.cnt, w.pts, w.pt_dp, w.pt_lastj,
                                                                   w.entry_dp, w.cont);
         }
-        if (ps.dp_last) k_dp_last<<<(unsigned)eb, DR_BLOCK, 0, hs>>>(w.q, w.cnt, w.q_cap, w.entry_dp, w.pt_lastj, w.pt_dp);
+        if (ps.dp_last) k_dp_last<<<1024, DR_BLOCK, 0, hs>>>(w.q, w.cnt, w.q_cap, w.entry_dp, w.pt_lastj, w.pt_dp);
         {
             LaunchTimer t(tm, TK_DP, hs);
             k_dp<MAXB><<<(unsigned)ps.nblocks, DR_BLOCK, 0, hs>>>(w.jobs, R, nr, w.pts, w.pt_dp, w.counts);
@@ -2187,15 +2382,13 @@ static dr_status run_noalloc(const Plan &P, Workspace &w, hipStream_t hs) {
                 part = std::max(1ll, std::min((f1 - f0) / 2, (long long)(0.9 * (double)w.q_cap / per)));
                 continue;
             }
-            long long eb = resident_blocks(k_edge<MAXB>, g_edge_blocks[MAXB == 1 ? 0 : MAXB == 2 ? 1 : MAXB == 4 ? 2 : 3]);
-            k_edge<MAXB><<<(unsigned)eb, DR_BLOCK, 0, hs>>>(w.jobs, w.q, w.cnt, w.q_cap, w.pts, w.pt_dp, w.pt_lastj,
-                                                            w.entry_dp, w.cont);
+            launch_edge_trace(w, hs);
             long long sb = resident_blocks(k_edge_shade<MAXB>,
                                            g_shade_blocks[MAXB == 1 ? 0 : MAXB == 2 ? 1 : MAXB == 4 ? 2 : 3]);
             k_edge_shade<MAXB><<<(unsigned)sb, DR_BLOCK, 0, hs>>>(w.jobs, w.q, w.cnt, w.pts, w.pt_dp, w.pt_lastj,
                                                                   w.entry_dp, w.cont);
             if (ps.dp_last)
-                k_dp_last<<<(unsigned)eb, DR_BLOCK, 0, hs>>>(w.q, w.cnt, w.q_cap, w.entry_dp, w.pt_lastj, w.pt_dp);
+                k_dp_last<<<1024, DR_BLOCK, 0, hs>>>(w.q, w.cnt, w.q_cap, w.entry_dp, w.pt_lastj, w.pt_dp);
             f0 = f1;
             if (per > 0.0) part = std::max(1ll, (long long)(0.9 * (double)w.q_cap / per));
         }
