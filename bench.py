@@ -641,7 +641,8 @@ def gpu_leg(w, steps, warmup, calibrate=False):
     n_points = samples * nb
     bytes_k["select"] += (B_POINT * n_points + B_TREE_EXPAND * cb["edge_nodes_visited"] +
                           B_EDGE_TEST * cb["edges_tested"] + B_QUEUE * cb["secondary_edges"])
-    # the edge samples run in two launches per pass (k_edge_draw and k_edge_trace, then k_edge_shade
+    # the edge samples run in two parts per pass (k_edge_draw and k_edge_trace,
+    # timed together, then k_edge_shade
     # on the samples with continuation paths): their work counters are one
     # figure, so their times are taken together as "edge"
     kt["edge_shade_ms"] = kt["shade_ms"]
