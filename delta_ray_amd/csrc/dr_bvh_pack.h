@@ -4,58 +4,60 @@
 #include "dr_math.h"
 #include "dr_types.h"
 
-// The grid over the root's box: 16-bit coordinate q = (v - lo) * scale + 2, so
-// that the box spans 2 .. 65533 and rounding outward stays within 16 bits.
-// Axes without extent get a thousandth of the largest one's.
-struct BvhGrid {
-    float lo[3], scale[3], rscale[3];
+// One axis of a node's frame: planes at origin + q * step, q = 0 .. 255, the step
+// as the exponent bits of a float.
+// The step is the least power of two of which 252 span both boxes, and at least
+// two units in the last place of the largest coordinate, so that the origin,
+// one step below the boxes, rounds by at most half a step.  An axis with
+// coordinates that are not finite, or too large for sums of them, has the origin
+// not-a-number: so are all of its distances, and it does not constrain a ray.
+struct PackAxis {
+    float origin, rstep;
+    uint32_t exponent;
 };
-DR_INLINE BvhGrid bvh_grid(const DrNode &root) {
-    const float l[2][3] = {{root.a[0], root.a[1], root.a[2]}, {root.b[2], root.b[3], root.c[0]}};
-    const float h[2][3] = {{root.a[3], root.b[0], root.b[1]}, {root.c[1], root.c[2], root.c[3]}};
-    BvhGrid g;
-    float ext[3], most = 0.f;
-    for (int k = 0; k < 3; k++) {
-        g.lo[k] = fminf(l[0][k], l[1][k]);
-        ext[k] = fmaxf(h[0][k], h[1][k]) - g.lo[k];
-        most = fmaxf(most, ext[k]);
-    }
-    for (int k = 0; k < 3; k++) {
-        float e = fmaxf(fmaxf(ext[k], 1e-3f * most), 1e-18f);
-        g.scale[k] = fminf(65531.f / e, 1e20f);
-        g.rscale[k] = 1.f / g.scale[k];
-    }
-    return g;
+DR_INLINE PackAxis pack_axis(float lo, float hi) {
+    float most = fmaxf(fabsf(lo), fabsf(hi)), ext = hi - lo;
+    if (!(lo <= hi && most < 1e36f)) return PackAxis{__uint_as_float(0x7fc00000u), 0.f, 127u};
+    uint32_t b = __float_as_uint(fmaxf(fmaxf(ext * (1.f / 252.f), most * 2.384185791015625e-7f), 1e-30f));
+    uint32_t e = (b >> 23) + ((b & 0x7fffffu) != 0);
+    return PackAxis{lo - __uint_as_float(e << 23), __uint_as_float((254u - e) << 23), e};
 }
-// a lower / upper plane on the grid, at least one step outward (not-a-number:
-// the grid's end); an empty slot (lo = +inf, hi = -inf) stays empty
-DR_INLINE uint32_t pack_lo(float v, float lo, float scale) {
-    float q = (v - lo) * scale + 2.f;
-    if (!(q >= 1.f)) return 0u;
-    return q >= 65536.f ? 65535u : (uint32_t)(floorf(q) - 1.f);
+// a lower / upper plane on the axis, at least a 64th of a step outside v: the
+// walk's rounding is at most 1e-4 of a step near the box (not-a-number: any)
+DR_INLINE uint32_t pack_lo(float v, const PackAxis &a) {
+    return (uint32_t)fminf(fmaxf(floorf((v - a.origin) * a.rstep - 0.015625f), 0.f), 255.f);
 }
-DR_INLINE uint32_t pack_hi(float v, float lo, float scale) {
-    float q = (v - lo) * scale + 2.f;
-    if (!(q <= 65534.f)) return 65535u;
-    return q <= -1.f ? 0u : (uint32_t)(ceilf(q) + 1.f);
+DR_INLINE uint32_t pack_hi(float v, const PackAxis &a) {
+    return (uint32_t)fminf(fmaxf(ceilf((v - a.origin) * a.rstep + 0.015625f), 0.f), 255.f);
 }
-DR_INLINE DrPackedNode pack_node(const DrNode &n, const BvhGrid &g) {
-    const float l[2][3] = {{n.a[0], n.a[1], n.a[2]}, {n.b[2], n.b[3], n.c[0]}};
-    const float h[2][3] = {{n.a[3], n.b[0], n.b[1]}, {n.c[1], n.c[2], n.c[3]}};
+// Node i of a tree in depth-first order (drh::bvh_in_order()): an interior left
+// child is node i + 1, as is an interior right one beside a leaf (the two then
+// change places: the first child is a leaf only if both are), and sibling
+// leaves' triangles lie side by side.
+DR_INLINE DrPackedNode pack_node(const DrNode &n, int i) {
+    const bool leaf0 = n.d[2] > 0, leaf1 = n.d[3] > 0;
+    // a root that is a leaf has no sibling: the second leaf has no triangles
+    const bool none = !leaf1 && n.d[1] == 0;
+    const bool swap = leaf0 && !leaf1 && !none;
     DrPackedNode p;
-    for (int k = 0; k < 3; k++) {
-        p.w[k] = pack_lo(l[0][k], g.lo[k], g.scale[k]) | pack_lo(l[1][k], g.lo[k], g.scale[k]) << 16;
-        p.w[3 + k] = pack_hi(h[0][k], g.lo[k], g.scale[k]) | pack_hi(h[1][k], g.lo[k], g.scale[k]) << 16;
-    }
-    for (int c = 0; c < 2; c++)
-        p.w[6 + c] = (uint32_t)(n.d[2 + c] > 0 ? ~(2 * n.d[c] + (n.d[2 + c] - 1)) : n.d[c]);
-    return p;
-}
-// element `i` of the head: the grid's nine floats
-DR_INLINE DrPackedNode pack_head(const BvhGrid &g, int i) {
-    const float f[16] = {g.lo[0], g.lo[1], g.lo[2], g.scale[0], g.scale[1], g.scale[2], g.rscale[0], g.rscale[1],
-                         g.rscale[2], 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    DrPackedNode p;
-    for (int k = 0; k < 8; k++) p.w[k] = __float_as_uint(f[8 * i + k]);
+    uint32_t exps = 0;
+    auto boxes = [&](int k, float l0, float h0, float l1, float h1) {
+        if (none) {
+            l1 = l0;
+            h1 = h0;
+        }
+        // (not-a-number in either box: `lo <= hi` fails)
+        const PackAxis a = pack_axis(l1 < l0 || l1 != l1 ? l1 : l0, h1 > h0 || h1 != h1 ? h1 : h0);
+        const uint32_t c0 = pack_lo(l0, a) | pack_hi(h0, a) << 8, c1 = pack_lo(l1, a) | pack_hi(h1, a) << 8;
+        p.w[k] = __float_as_uint(a.origin);
+        p.w[4 + k] = swap ? c1 | c0 << 16 : c0 | c1 << 16;
+        exps |= a.exponent << (23 - 8 * k);
+    };
+    boxes(0, n.a[0], n.a[3], n.b[2], n.c[1]);
+    boxes(1, n.a[1], n.b[0], n.b[3], n.c[2]);
+    boxes(2, n.a[2], n.b[1], n.c[0], n.c[3]);
+    const uint32_t n0 = leaf0 && !swap ? (uint32_t)n.d[2] : 0u, n1 = leaf1 ? (uint32_t)n.d[3] : (swap ? (uint32_t)n.d[2] : 0u);
+    p.w[3] = exps | (n0 > 0 ? 0x80000000u : 0u) | (leaf0 || leaf1 ? 1u : 0u) | n0 << 1 | n1 << 3;
+    p.w[7] = (uint32_t)(leaf0 ? n.d[0] : n.d[1]);
     return p;
 }

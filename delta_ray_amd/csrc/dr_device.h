@@ -47,60 +47,73 @@ DR_INLINE bool tri_hit(const DrTri &T, F3 org, F3 dir, float tmin, float tmax, f
     return u >= 0.f && v >= 0.f && u + v <= 1.f && t > tmin && t < tmax;
 }
 
-// A ray on the grid of the packed boxes: t = (q - org) * inv.  An axis the ray
-// does not move along (1 / dir infinite) does not constrain the interval: its
-// factor is 0 and its offset takes the slab distances to -inf and +inf.
-struct BoxRay {
-    F3 org, inv, off;
-};
-DR_INLINE BoxRay box_ray(const DrSceneView &S, F3 org, F3 dir) {
-    const DR_GLOBAL float4 *g = (const DR_GLOBAL float4 *)S.packed;
-    const float4 A = g[0], B = g[1], C = g[2];  // lo, scale, 1 / scale
-    BoxRay r;
-    r.org = F3{(org.x - A.x) * A.w + 2.f, (org.y - A.y) * B.x + 2.f, (org.z - A.z) * B.y + 2.f};
-    F3 i = F3{1.f / dir.x, 1.f / dir.y, 1.f / dir.z};
-    bool px = fabsf(i.x) == DR_INF, py = fabsf(i.y) == DR_INF, pz = fabsf(i.z) == DR_INF;
-    r.inv = F3{px ? 0.f : i.x * B.z, py ? 0.f : i.y * B.w, pz ? 0.f : i.z * C.x};
-    r.off = F3{px ? -DR_INF : 0.f, py ? -DR_INF : 0.f, pz ? -DR_INF : 0.f};
-    return r;
+// 1 / direction of a ray, for box tests.  An axis the ray does not move along
+// (1 / dir infinite) does not constrain the interval: its factor is
+// not-a-number, which minima and maxima over the axes pass over.
+DR_INLINE F3 box_inv(F3 dir) {
+    auto rcp = [](float d) {
+        float i = 1.f / d;
+        return fabsf(i) == DR_INF ? __uint_as_float(0x7fc00000u) : i;
+    };
+    return F3{rcp(dir.x), rcp(dir.y), rcp(dir.z)};
 }
 // A packed node as it is fetched.
 struct NodeFetch {
     uint4 P, Q;
+    int next;
     DR_INLINE NodeFetch(const DrSceneView &S, int node) {
-        const DR_GLOBAL uint4 *n = (const DR_GLOBAL uint4 *)(S.packed + DR_PACKED_HEAD + node);
+        const DR_GLOBAL uint4 *n = (const DR_GLOBAL uint4 *)(S.packed + node);
         P = n[0];
         Q = n[1];
+        next = node + 1;
     }
-    DR_INLINE int child(int c) const { return (int)(c ? Q.w : Q.z); }
+    DR_INLINE bool leaf(int c) const { return c == 0 ? (int)P.w < 0 : (P.w & 1u) != 0; }
+    // the child's node
+    DR_INLINE int child(int c) const { return c == 0 ? next : (int)Q.w; }
+    // the triangles of the leaves among the children that are on: slots first .. end - 1
+    DR_INLINE void leaves(bool on0, bool on1, int &first, int &end) const {
+        const uint32_t n0 = (P.w >> 1) & 3u, n1 = (P.w >> 3) & 3u;
+        first = (int)(Q.w + (on0 ? 0u : n0));
+        end = (int)(Q.w + n0 + (on1 ? n1 : 0u));
+    }
 };
-DR_INLINE int leaf_first(int code) { return ~code >> 1; }
-DR_INLINE int leaf_count(int code) { return (~code & 1) + 1; }
+// A ray's distances to the planes of a node's frame: t = q * step + org.
+struct FrameRay {
+    F3 step, org;
+    DR_INLINE FrameRay(const NodeFetch &N, F3 o, F3 inv) {
+        auto power = [&](int k) { return __uint_as_float((N.P.w << (8 * k)) & 0x7f800000u); };
+        step = F3{power(0) * inv.x, power(1) * inv.y, power(2) * inv.z};
+        org = F3{(__uint_as_float(N.P.x) - o.x) * inv.x, (__uint_as_float(N.P.y) - o.y) * inv.y,
+                 (__uint_as_float(N.P.z) - o.z) * inv.z};
+    }
+};
 // Slab test of child c's box, widened by a relative 1e-5 (+1e-7) so that
 // rounding can never hide a triangle the exact test would accept: the planes
-// lie at least one grid step outside the exact box, which covers the rounding
-// of org near the grid, and the relative part covers it far away and that of
-// the factors.  The widening is monotone, so the entry and exit are widened
-// once, after the max / min over the axes.
+// lie at least a 64th of a step outside the exact box.  Within 512 steps of the
+// frame the rounding of the distances is below 1e-4 of a step, and beyond it
+// below 5e-7 of the distance.  The widening is monotone, so the entry and exit
+// are widened once, after the max / min over the axes.
 //
 // Ray walks are bound by the latency and bytes of their node loads (16-byte
 // loads, a cache line per lane): with 32-byte nodes instead of 64-byte ones,
-// and both boxes tested before any leaf, a forward render of the 32 k triangle
-// heightfield (16.8 M samples) takes 6.7 ms instead of 8.6, a million plain rays 226
-// us instead of 334, and its adjoint render 232 instead of 252 ms.
-DR_INLINE bool box_hit(const NodeFetch &N, int c, const BoxRay &r, float tmin, float tmax, float &tenter) {
-    auto q = [&](uint32_t w) { return (float)(c ? w >> 16 : w & 0xffffu); };
-    const float lx = q(N.P.x), ly = q(N.P.y), lz = q(N.P.z), hx = q(N.P.w), hy = q(N.Q.x), hz = q(N.Q.y);
-    float ax = fmaf(lx - r.org.x, r.inv.x, r.off.x), bx = fmaf(hx - r.org.x, r.inv.x, -r.off.x);
-    float ay = fmaf(ly - r.org.y, r.inv.y, r.off.y), by = fmaf(hy - r.org.y, r.inv.y, -r.off.y);
-    float az = fmaf(lz - r.org.z, r.inv.z, r.off.z), bz = fmaf(hz - r.org.z, r.inv.z, -r.off.z);
+// and sibling leaves' triangles in one loop that loads ahead, a forward render
+// of the 32 k triangle heightfield (16.8 M samples) takes 6.8 ms instead of 8.6
+// and a million plain rays 212 us instead of 334.  Planes on one grid over the
+// whole scene would be simpler and as fast on these scenes, but a ground quad
+// 1000 times a mesh's size makes its rays visit twice the nodes, and one 100 000
+// times its size 600 times.
+DR_INLINE bool box_hit(const NodeFetch &N, int c, const FrameRay &f, float tmin, float tmax, float &tenter) {
+    auto lo = [&](uint32_t w) { return (float)(c ? (w >> 16) & 0xffu : w & 0xffu); };
+    auto hi = [&](uint32_t w) { return (float)(c ? w >> 24 : (w >> 8) & 0xffu); };
+    float ax = fmaf(lo(N.Q.x), f.step.x, f.org.x), bx = fmaf(hi(N.Q.x), f.step.x, f.org.x);
+    float ay = fmaf(lo(N.Q.y), f.step.y, f.org.y), by = fmaf(hi(N.Q.y), f.step.y, f.org.y);
+    float az = fmaf(lo(N.Q.z), f.step.z, f.org.z), bz = fmaf(hi(N.Q.z), f.step.z, f.org.z);
     float mn = fmaxf(fmaxf(fminf(ax, bx), fminf(ay, by)), fminf(az, bz));
     float mx = fminf(fminf(fmaxf(ax, bx), fmaxf(ay, by)), fmaxf(az, bz));
     mn = fmaf(fabsf(mn), -1e-5f, mn) - 1e-7f;
     mx = fmaf(fabsf(mx), 1e-5f, mx) + 1e-7f;
     tenter = fmaxf(mn, tmin);
-    // (an empty slot, lo above hi, never hits)
-    return tenter <= fminf(mx, tmax) && lx <= hx;
+    return tenter <= fminf(mx, tmax);
 }
 
 // Optional counters (rays, nodes visited, triangles tested) for the roofline
@@ -147,7 +160,7 @@ struct TraceStack {
 DR_INLINE Isect trace_closest(const DrSceneView &S, F3 org, F3 dir, float tmin, float tmax, float &ou, float &ov) {
     Isect best = no_hit();
     if (S.num_nodes == 0) return best;
-    const BoxRay r = box_ray(S, org, dir);
+    const F3 inv = box_inv(dir);
     float best_t = tmax;
     int best_g = -1;
     float bu = 0.f, bv = 0.f;
@@ -160,15 +173,20 @@ DR_INLINE Isect trace_closest(const DrSceneView &S, F3 org, F3 dir, float tmin, 
     const uint32_t cap = 2u * (uint32_t)S.num_nodes + 8u;
     while (nn < cap) {
         const NodeFetch N(S, node);
-        const int c0 = N.child(0), c1 = N.child(1);
         nn++;
+        const FrameRay f(N, org, inv);
         float t0, t1;
-        bool h0 = box_hit(N, 0, r, tmin, best_t, t0);
-        bool h1 = box_hit(N, 1, r, tmin, best_t, t1);
-        // leaves first
-        if (h0 && c0 < 0) {
-            for (int i = 0, k = leaf_count(c0); i < k; i++) {
-                const DrTri T = gptr(S.tris)[leaf_first(c0) + i];
+        bool h0 = box_hit(N, 0, f, tmin, best_t, t0);
+        bool h1 = box_hit(N, 1, f, tmin, best_t, t1);
+        // leaves first (the first child is a leaf only if both are)
+        if ((h0 && N.leaf(0)) || (h1 && N.leaf(1))) {
+            int i, end;
+            N.leaves(h0 && N.leaf(0), h1, i, end);
+            // (the next triangle is on its way while one is tested)
+            DrTri next = gptr(S.tris)[min(i, end - 1)];
+            while (i < end) {
+                const DrTri T = next;
+                next = gptr(S.tris)[min(++i, end - 1)];
                 float u, v, t;
                 nt++;
                 if (tri_hit(T, org, dir, tmin, tmax, u, v, t)) {
@@ -178,34 +196,21 @@ DR_INLINE Isect trace_closest(const DrSceneView &S, F3 org, F3 dir, float tmin, 
                     }
                 }
             }
-            h0 = false;
-        }
-        if (h1 && c1 < 0) {
-            for (int i = 0, k = leaf_count(c1); i < k; i++) {
-                const DrTri T = gptr(S.tris)[leaf_first(c1) + i];
-                float u, v, t;
-                nt++;
-                if (tri_hit(T, org, dir, tmin, tmax, u, v, t)) {
-                    int g = __float_as_int(T.v0[3]);
-                    if (best_g < 0 || t < best_t || (t == best_t && g < best_g)) {
-                        best_t = t; best_g = g; bu = u; bv = v;
-                    }
-                }
-            }
+            h0 = h0 && !N.leaf(0) && t0 <= best_t;
             h1 = false;
         }
         if (h0 && h1) {
-            int near = c0, far = c1;
-            if (t1 < t0) { near = c1; far = c0; }
+            int near = N.child(0), far = N.child(1);
+            if (t1 < t0) { near = N.child(1); far = N.child(0); }
             // the builder bounds the depth, so the stack cannot fill; a full
             // stack would be counted, not silently dropped
             if (sp < DR_STACK) stack.put(sp++, far);
             else if (S.stats) atomicAdd(&S.stats[7], 1ull);
             node = near;
         } else if (h0) {
-            node = c0;
+            node = N.child(0);
         } else if (h1) {
-            node = c1;
+            node = N.child(1);
         } else {
             if (sp == 0) break;
             node = stack.get(--sp);
@@ -224,17 +229,17 @@ DR_INLINE Isect trace_closest(const DrSceneView &S, F3 org, F3 dir, float tmin, 
 
 // Closest hits of two rays from one origin in one walk of the BVH (the two
 // side rays of an edge sample are a few 1e-3 rad apart and visit nearly the
-// same nodes, so one node fetch serves both).  A node is entered when either
-// ray's box test passes; each ray keeps its own closest hit and makes its
+// same nodes, so one node fetch serves both).  A node or leaf is entered when
+// either ray's box test passes; each ray keeps its own closest hit and makes its
 // own box and triangle tests with trace_closest's arithmetic and tie rule.
 // Culling with a ray's current closest distance is conservative and the
-// closest hit does not depend on the visiting order, so each result is the
-// one trace_closest returns for that ray.  The walk is a state advanced one
+// closest hit depends neither on the visiting order nor on further triangles
+// tested, so each result is the one trace_closest returns for that ray.  The walk is a state advanced one
 // node at a time, so that a kernel can give a lane new rays as soon as its
 // walk ends.
 struct Walk2 {
     F3 org, da, db;
-    BoxRay ra, rb;
+    F3 ia, ib;     // 1 / da, 1 / db (box_inv)
     float ta, tb;  // closest distances so far
     int ga, gb;    // their triangles (global ids, -1: none)
     int node, sp;
@@ -249,8 +254,8 @@ struct Walk2 {
             nn = nt = 0;
             return false;
         }
-        ra = box_ray(S, org, da);
-        rb = box_ray(S, org, db);
+        ia = box_inv(da);
+        ib = box_inv(db);
         ta = tb = DR_INF;
         ga = gb = -1;
         node = sp = 0;
@@ -261,53 +266,49 @@ struct Walk2 {
     DR_INLINE bool step(const DrSceneView &S, TraceStack &stack) {
         const float tmin = 1e-3f;
         const NodeFetch N(S, node);
-        const int c0 = N.child(0), c1 = N.child(1);
         nn++;
-        auto test = [&](int first, int count, bool a_on, bool b_on) {
-            for (int i = 0; i < count; i++) {
-                const DrTri T = gptr(S.tris)[first + i];
+        const FrameRay fa(N, org, ia), fb(N, org, ib);
+        float a0, a1, b0, b1;
+        bool ha0 = box_hit(N, 0, fa, tmin, ta, a0);
+        bool ha1 = box_hit(N, 1, fa, tmin, ta, a1);
+        bool hb0 = box_hit(N, 0, fb, tmin, tb, b0);
+        bool hb1 = box_hit(N, 1, fb, tmin, tb, b1);
+        bool h0 = ha0 || hb0, h1 = ha1 || hb1;
+        // leaves first (the first child is a leaf only if both are)
+        if ((h0 && N.leaf(0)) || (h1 && N.leaf(1))) {
+            int i, end;
+            N.leaves(h0 && N.leaf(0), h1, i, end);
+            for (; i < end; i++) {
+                const DrTri T = gptr(S.tris)[i];
                 int g = __float_as_int(T.v0[3]);
                 float u, v, t;
                 nt++;
-                if (a_on && tri_hit(T, org, da, tmin, DR_INF, u, v, t) &&
-                    (ga < 0 || t < ta || (t == ta && g < ga))) {
+                if (tri_hit(T, org, da, tmin, DR_INF, u, v, t) && (ga < 0 || t < ta || (t == ta && g < ga))) {
                     ta = t; ga = g;
                 }
-                if (b_on && tri_hit(T, org, db, tmin, DR_INF, u, v, t) &&
-                    (gb < 0 || t < tb || (t == tb && g < gb))) {
+                if (tri_hit(T, org, db, tmin, DR_INF, u, v, t) && (gb < 0 || t < tb || (t == tb && g < gb))) {
                     tb = t; gb = g;
                 }
             }
-        };
-        float a0, a1, b0, b1;
-        bool ha0 = box_hit(N, 0, ra, tmin, ta, a0);
-        bool ha1 = box_hit(N, 1, ra, tmin, ta, a1);
-        bool hb0 = box_hit(N, 0, rb, tmin, tb, b0);
-        bool hb1 = box_hit(N, 1, rb, tmin, tb, b1);
-        bool h0 = ha0 || hb0, h1 = ha1 || hb1;
-        // leaves first
-        if (h0 && c0 < 0) {
-            test(leaf_first(c0), leaf_count(c0), ha0, hb0);
-            h0 = false;
-        }
-        if (h1 && c1 < 0) {
-            test(leaf_first(c1), leaf_count(c1), ha1, hb1);
+            ha0 = ha0 && a0 <= ta;
+            hb0 = hb0 && b0 <= tb;
+            h0 = !N.leaf(0) && (ha0 || hb0);
             h1 = false;
         }
         if (h0 && h1) {
             // nearer child first, by the first ray that enters both
             float t0 = ha0 && ha1 ? a0 : b0, t1 = ha0 && ha1 ? a1 : b1;
-            int near = c0, far = c1;
-            if (t1 < t0) { near = c1; far = c0; }
+            int near = N.child(0), far = N.child(1);
+            if (t1 < t0) { near = N.child(1); far = N.child(0); }
             // the builder bounds the depth, so the stack cannot fill; a full
             // stack would be counted, not silently dropped
             if (sp < DR_STACK) stack.put(sp++, far);
             else if (S.stats) atomicAdd(&S.stats[7], 1ull);
             node = near;
         } else if (h0) {
-            node = c0;
+            node = N.child(0);
         } else if (h1) {
-            node = c1;
+            node = N.child(1);
         } else {
             if (sp == 0) return false;
             node = stack.get(--sp);
@@ -327,7 +328,7 @@ struct Walk2 {
 
 DR_INLINE bool trace_any(const DrSceneView &S, F3 org, F3 dir, float tmin, float tmax) {
     if (S.num_nodes == 0) return false;
-    const BoxRay r = box_ray(S, org, dir);
+    const F3 inv = box_inv(dir);
     TraceStack stack;
     int sp = 0;
     int node = 0;
@@ -336,38 +337,34 @@ DR_INLINE bool trace_any(const DrSceneView &S, F3 org, F3 dir, float tmin, float
     const uint32_t cap = 2u * (uint32_t)S.num_nodes + 8u;
     while (nn < cap) {
         const NodeFetch N(S, node);
-        const int c0 = N.child(0), c1 = N.child(1);
         nn++;
+        const FrameRay f(N, org, inv);
         float t0, t1;
-        bool h0 = box_hit(N, 0, r, tmin, tmax, t0);
-        bool h1 = box_hit(N, 1, r, tmin, tmax, t1);
-        if (h0 && c0 < 0) {
-            for (int i = 0, k = leaf_count(c0); i < k && !hit; i++) {
+        bool h0 = box_hit(N, 0, f, tmin, tmax, t0);
+        bool h1 = box_hit(N, 1, f, tmin, tmax, t1);
+        if ((h0 && N.leaf(0)) || (h1 && N.leaf(1))) {
+            int i, end;
+            N.leaves(h0 && N.leaf(0), h1, i, end);
+            DrTri next = gptr(S.tris)[min(i, end - 1)];
+            while (i < end && !hit) {
+                const DrTri T = next;
+                next = gptr(S.tris)[min(++i, end - 1)];
                 float u, v, t;
                 nt++;
-                const DrTri T = gptr(S.tris)[leaf_first(c0) + i];
                 hit = tri_hit(T, org, dir, tmin, tmax, u, v, t);
             }
-            h0 = false;
-        }
-        if (h1 && c1 < 0 && !hit) {
-            for (int i = 0, k = leaf_count(c1); i < k && !hit; i++) {
-                float u, v, t;
-                nt++;
-                const DrTri T = gptr(S.tris)[leaf_first(c1) + i];
-                hit = tri_hit(T, org, dir, tmin, tmax, u, v, t);
-            }
+            h0 = h0 && !N.leaf(0);
             h1 = false;
         }
         if (hit) break;
         if (h0 && h1) {
-            if (sp < DR_STACK) stack.put(sp++, c1);
+            if (sp < DR_STACK) stack.put(sp++, N.child(1));
             else if (S.stats) atomicAdd(&S.stats[7], 1ull);
-            node = c0;
+            node = N.child(0);
         } else if (h0) {
-            node = c0;
+            node = N.child(0);
         } else if (h1) {
-            node = c1;
+            node = N.child(1);
         } else {
             if (sp == 0) break;
             node = stack.get(--sp);

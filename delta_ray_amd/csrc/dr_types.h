@@ -4,7 +4,7 @@
 // HBM layout (all arrays 16-byte aligned, one allocation per array):
 //   nodes      BVH2 nodes, 64 B: both child boxes in the parent (refits)
 //   packed     the same nodes as ray walks read them, 32 B: both child boxes
-//              on a 16-bit grid, so one fetch of 32 B tests two boxes
+//              in bytes on the node's own frame, so one fetch tests two boxes
 //   tris       48 B per triangle in leaf order: v0, e1 = v1-v0, e2 = v2-v0
 //              (float4 each; v0.w carries the global triangle id)
 //   verts      float3 per global vertex (all shapes concatenated)
@@ -37,17 +37,17 @@ struct DrNode {
     int d[4];
 };
 
-// What ray walks read of a node: the planes of both child boxes on a 16-bit
-// grid over the root's box, rounded outward by at least one step, so that a
-// packed box holds the exact one; half the bytes of a DrNode.  w[0..5]: lo x, y,
-// z, hi x, y, z of child 0 (low half) and child 1 (high half); w[6], w[7]: the
-// children, node index or ~(2 * first triangle slot + count - 1) for a leaf
-// (the builders make leaves of one or two triangles).  The array starts with
-// the grid (DR_PACKED_HEAD elements): lo[3], scale[3], 1 / scale[3].
+// What ray walks read of a node: the planes of both child boxes in bytes, on a
+// frame of the node's own (dr_bvh_pack.h), so that a box is wider than the
+// exact one by at most about a hundredth of its parent's at any scale of the
+// scene; half the bytes of a DrNode.  w[0..2]: the frame's origin; w[3]: its
+// steps' exponents (x in bits 23-30, y 15-22, z 7-14), bit 31 / 0: child 0 / 1 is
+// a leaf, bits 1-2 / 3-4: triangles of leaf 0 / 1 (0: not a leaf); w[4..6]: per
+// axis lo and hi of child 0, then of child 1; w[7]: the first triangle slot of
+// the leaves, or child 1's node.  Child 0's node is the next one.
 struct alignas(16) DrPackedNode {
     uint32_t w[8];
 };
-#define DR_PACKED_HEAD 2
 
 struct DrTri {
     float v0[4];  // w: global triangle id (int bits)

@@ -55,8 +55,7 @@ struct PrimaryOut {
     float *func_int;      // device: the distribution's integral
 };
 
-// the packed copy of a BVH's nodes (dr_bvh_pack.h); packed: n + DR_PACKED_HEAD
-// elements
+// the packed copy of a BVH's nodes (dr_bvh_pack.h), n elements
 void pack_bvh(const DrNode *nodes, int n, DrPackedNode *packed, hipStream_t st);
 // triangle records and BVH boxes
 void refit_geometry(const RefitView &v, hipStream_t st);

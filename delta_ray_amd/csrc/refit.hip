@@ -450,10 +450,7 @@ static unsigned grid(long long n, int b) { return (unsigned)((n + b - 1) / b); }
 __global__ void k_pack_bvh(const DrNode *__restrict__ nodes, int n, DrPackedNode *__restrict__ packed) {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    const BvhGrid g = bvh_grid(nodes[0]);
-    if (i == 0)
-        for (int k = 0; k < DR_PACKED_HEAD; k++) packed[k] = pack_head(g, k);
-    packed[DR_PACKED_HEAD + i] = pack_node(nodes[i], g);
+    packed[i] = pack_node(nodes[i], i);
 }
 void pack_bvh(const DrNode *nodes, int n, DrPackedNode *packed, hipStream_t st) {
     if (n > 0) k_pack_bvh<<<grid(n, RF_BLOCK), RF_BLOCK, 0, st>>>(nodes, n, packed);

@@ -1704,7 +1704,7 @@ static bool upload_structures(dr_scene *s) {
     v.packed = nullptr;
     if (v.num_nodes > 0) {
         void *pn = nullptr;
-        if (!alloc_to(A, (hs.nodes.size() + DR_PACKED_HEAD) * sizeof(DrPackedNode), &pn)) return false;
+        if (!alloc_to(A, hs.nodes.size() * sizeof(DrPackedNode), &pn)) return false;
         v.packed = (decltype(v.packed))pn;
         drrefit::pack_bvh((const DrNode *)v.nodes, v.num_nodes, (DrPackedNode *)pn, nullptr);
         // (renders may run on streams that do not wait for this one)

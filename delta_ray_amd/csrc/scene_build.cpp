@@ -740,6 +740,18 @@ void tree_levels(int n, Children children, std::vector<int> &order, std::vector<
 }
 }  // namespace
 
+bool bvh_in_order(const std::vector<DrNode> &nodes) {
+    for (int i = 0; i < (int)nodes.size(); i++) {
+        const int *d = nodes[i].d;
+        bool leaf0 = d[2] > 0, leaf1 = d[3] > 0, none = !leaf1 && d[1] == 0;
+        if (d[2] > 2 || d[3] > 2) return false;
+        if (!leaf0 && d[0] != i + 1) return false;
+        if (leaf0 && leaf1 && d[1] != d[0] + d[2]) return false;
+        if (leaf0 && !leaf1 && !none && d[1] != i + 1) return false;
+    }
+    return true;
+}
+
 std::string adopt_device_bvh(HostScene &hs, const std::vector<DrNode> &built, std::vector<DrTri> &tris) {
     int m = (int)built.size();
     if (m == 0) return "empty device BVH";
@@ -775,6 +787,7 @@ std::string adopt_device_bvh(HostScene &hs, const std::vector<DrNode> &built, st
     // the ray traversal stack holds at most one far child per interior level
     int levels = (int)off.size() - 1;
     if (levels > DR_STACK) return "device BVH deeper than the traversal stack";
+    if (!bvh_in_order(nodes)) return "device BVH is not in depth-first order";
     hs.nodes.swap(nodes);
     hs.tris.swap(tris);
     hs.bvh_lv.swap(lv);
@@ -834,6 +847,7 @@ std::string build_structures(HostScene &hs) {
         return "edge tree deeper than the traversal stack";
     // the ray traversal stack holds at most one far child per interior level
     if (hs.bvh_depth > DR_STACK) return "triangle BVH deeper than the traversal stack";
+    if (!bvh_in_order(hs.nodes)) return "triangle BVH is not in depth-first order";
     build_geo_records(hs);
     // refit tables: levels of the three trees, edge ranges of the edge-tree nodes
     tree_levels((int)hs.nodes.size(), [&](int i, int *c) {

@@ -68,6 +68,9 @@ void build_geo_records(HostScene &hs);
 // preorder, with refit levels.  Returns an empty string, or why it was
 // refused (the host tree is then kept).
 std::string adopt_device_bvh(HostScene &hs, const std::vector<DrNode> &built, std::vector<DrTri> &tris);
+// whether the BVH's nodes are in depth-first order and sibling leaves' triangles
+// lie side by side, at most two to a leaf, as packed nodes assume
+bool bvh_in_order(const std::vector<DrNode> &nodes);
 DrCamera make_camera(const dr_camera &c);
 void set_camera(HostScene &hs, const dr_camera &c);
 // Primary-edge list and distribution (pmf proportional to the clipped screen

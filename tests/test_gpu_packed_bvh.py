@@ -1,4 +1,4 @@
-"""Ray walks read boxes on a 16-bit grid over the scene (dr_bvh_pack.h), rounded
+"""Ray walks read boxes in bytes on a frame of each node's (dr_bvh_pack.h), rounded
 outward, so hits must stay those of a test of every triangle, bit for bit:
 scenes of one leaf and of many, tiny, huge, far from the origin and almost
 without extent along an axis (an offset that rounds the thin axis to a few
@@ -46,3 +46,61 @@ def test_hits_equal_brute_force(gpu, oracle, grid, scale, offset):
     np.testing.assert_array_equal(got[:, 0], ref[:, 0])
     np.testing.assert_array_equal(got[hit, 1:4], ref[hit, 1:4])
     assert hit.sum() > 300
+
+
+@pytest.mark.parametrize("tris", [1, 2, 3])
+def test_few_triangles(gpu, oracle, tris):
+    """a root that is one leaf, and the first tree with two"""
+    import torch
+    from delta_ray_amd import delta_ray as dr
+    m = workloads.diffuse_material([0.5, 0.5, 0.5])
+    v = np.array([[0, 0, 0], [1, 0, 0], [0, 1, 0], [1, 1, 0.5], [2, 1, 0]], np.float32)
+    s = dr.Shape(v, np.array([[0, 1, 2], [1, 3, 2], [1, 4, 3]], np.int32)[:tris], None, None, m, None)
+    s.light = dr.Light(s, np.ones(3, np.float32))
+    w = dict(camera=workloads.make_camera([0, 0, 3], [0, 0, 0], [0, 1, 0], 45.0, (8, 8)), shapes=[s], materials=[m],
+             lights=[s.light])
+    rng = np.random.default_rng(tris)
+    rays = np.zeros((4096, 8), np.float32)
+    rays[:, 0:2], rays[:, 2], rays[:, 3], rays[:, 7] = rng.uniform(-1, 3, (4096, 2)), 2.0, 1e-3, np.inf
+    rays[:, 4:7] = [0, 0, -1]
+    osc = oracle.scene_from_workload(w)
+    osc.use_bvh(False)
+    ref = osc.intersect(rays)
+    h = torch.zeros((4096, 4), dtype=torch.int32, device="cuda")
+    helpers.gpu_scene(w).intersect(torch.from_numpy(rays).cuda(), h)
+    got, hit = h.cpu().numpy(), ref[:, 0] >= 0
+    np.testing.assert_array_equal(got[:, 0], ref[:, 0])
+    np.testing.assert_array_equal(got[hit, 1:4], ref[hit, 1:4])
+    assert hit.sum() > 100
+
+
+@pytest.mark.parametrize("half", [1e2, 1e3, 1e5])
+def test_large_geometry_costs_no_visits(gpu, half):
+    """A ground quad of any size below a detailed mesh: the boxes around the mesh stay as
+    tight as with a quad of the mesh's size (1.3 times the visits: the top of the tree is
+    another one, which alone makes 1.05)."""
+    import torch
+    from delta_ray_amd import delta_ray as dr
+
+    def visits(h):
+        w = workloads.heightfield(grid=64, resolution=(16, 16))
+        v = np.array([[-h, -1, -h], [-h, -1, h], [h, -1, -h], [h, -1, h]], np.float32)
+        i = np.array([[0, 1, 2], [1, 3, 2]], np.int32)
+        w["shapes"].append(dr.Shape(v, i, None, None, w["materials"][0], None))
+        rng = np.random.default_rng(3)
+        rays = np.zeros((20000, 8), np.float32)
+        to = rng.uniform(-2, 2, (len(rays), 3))
+        to[:, 1] = 0
+        org = rng.normal(size=to.shape) * 4
+        org[:, 1] = np.abs(org[:, 1]) + 1
+        rays[:, 0:3], rays[:, 3] = org, 1e-3
+        rays[:, 4:7], rays[:, 7] = (to - org) / np.linalg.norm(to - org, axis=1, keepdims=True), np.inf
+        sc = helpers.gpu_scene(w)
+        sc.stats(True)
+        sc.intersect(torch.from_numpy(rays).cuda(), torch.zeros((len(rays), 4), dtype=torch.int32, device="cuda"))
+        st = sc.stats(False)
+        return st["nodes_visited"] / st["rays"], st["tris_visited"] / st["rays"]
+
+    nodes, tris = visits(half)
+    nodes0, tris0 = visits(5.0)
+    assert nodes < 1.3 * nodes0 and tris < 1.3 * tris0, (nodes, nodes0, tris, tris0)
