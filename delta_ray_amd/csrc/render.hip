@@ -214,7 +214,6 @@ DR_INLINE void sel_ctx(const SelPoint &P, const DrJob &J, EdgeTraversal &T, SPoi
     const DrSceneView &S = J.S;
     bool nrm = (P.info & 1) != 0;
     T.nodes = nrm ? S.nrm_nodes : S.sil_nodes;
-    T.edges = nrm ? S.nrm_edges : S.sil_edges;
     T.num_nodes = nrm ? S.num_nrm_nodes : S.num_sil_nodes;
     T.directional = nrm;
     T.B = P.B;
@@ -569,7 +568,6 @@ k_select(const DrJob *__restrict__ jobs, const int *list, const PointRec *pts, E
         uint32_t info = C[26 * 64 + pt];
         bool nrm = (info & 1) != 0;
         T.nodes = nrm ? J.S.nrm_nodes : J.S.sil_nodes;
-        T.edges = nullptr;
         T.num_nodes = nrm ? J.S.num_nrm_nodes : J.S.num_sil_nodes;
         T.directional = nrm;
         T.mode = LEARNED ? (int)(info >> 1) & 3 : 0;
@@ -681,6 +679,16 @@ k_select(const DrJob *__restrict__ jobs, const int *list, const PointRec *pts, E
         if (LEARNED) a = TreeAlt{__uint_as_float(x[SW - 2]), __uint_as_float(x[SW - 1])};
         return (x[0] >> 31) << 5 | (x[2] >> 31) << 4 | x[3] >> 28;
     };
+    // throttled() keeps room for every push; a stack that is full all the same
+    // would be counted, not silently dropped
+    auto push = [&](WaveStack<SW> &st, WaveSpill<SW> &spill, bool v, const uint32_t *x, uint32_t pt) {
+        if (st.push(v, x, lane, spill)) return;
+        int d0 = 0, d1 = 0;
+        half_count(v, pt, d0, d1);
+        out0 -= d0;
+        out1 -= d1;
+        if (jobs[job].S.stats && lane == 0) atomicAdd(&jobs[job].S.stats[7], (unsigned long long)(d0 + d1));
+    };
     // Fetches points until one is pending or none are left, then starts
     // pending points of one job.  False when nothing could be started now.
     auto start = [&]() -> bool {
@@ -753,7 +761,7 @@ k_select(const DrJob *__restrict__ jobs, const int *list, const PointRec *pts, E
         add_leaf(lf, rs.e, rs.a, pt);
         uint32_t x[SW];
         pack(x, rs.e, rs.a, pt);
-        cst.push(root && !lf, x, lane, cspill);
+        push(cst, cspill, root && !lf, x, pt);
         return true;
     };
 
@@ -791,8 +799,8 @@ k_select(const DrJob *__restrict__ jobs, const int *list, const PointRec *pts, E
             const bool leaf = v && c.nprims() > 0;
             const bool nc = CONE && et_need_cone(c, a);
             pack(x, c, a, pt);
-            if (CONE) cst.push(v && !leaf && nc, x, lane, cspill);
-            ast.push(v && !leaf && !nc, x, lane, aspill);
+            if (CONE) push(cst, cspill, v && !leaf && nc, x, pt);
+            push(ast, aspill, v && !leaf && !nc, x, pt);
             add_leaf(leaf, c, a, pt);
         };
         put(v0, c0, a0);
@@ -1283,8 +1291,8 @@ __global__ void k_intersect(DrSceneView S, const float *rays, long long n, int *
 // dr_test_tree_stack: every wave runs `ops` random pushes and pops of random
 // sets of its lanes on the selection kernel's wave stack, and keeps beside it
 // a plain array of what each position holds (position p: lane p % 64, element
-// p / 64 of its private array).  Odd waves carry 7 words per entry, even waves
-// 5; out[0] counts entries popped that differ, out[1] the deepest stack
+// p / 64 of its private array).  Odd waves carry 6 words per entry (the learned
+// mixture's), even waves 4; out[0] counts entries popped that differ, out[1] the deepest stack
 // reached, in entries per lane.
 template <int WORDS>
 DR_INLINE void tree_stack_run(long long ops, uint64_t seed, DR_LDS uint32_t *lds, unsigned long long *out) {
@@ -1346,11 +1354,59 @@ DR_INLINE void tree_stack_run(long long ops, uint64_t seed, DR_LDS uint32_t *lds
     atomicMax(&out[1], (unsigned long long)deepest);
 }
 __global__ void __launch_bounds__(DR_BLOCK) k_tree_stack(long long ops, uint64_t seed, unsigned long long *out) {
-    __shared__ uint32_t s_stack[7 * DR_WSTACK_LDS * (DR_BLOCK / 64)];
+    __shared__ uint32_t s_stack[6 * DR_WSTACK_LDS * (DR_BLOCK / 64)];
     const int w = threadIdx.x >> 6;
-    DR_LDS uint32_t *lds = (DR_LDS uint32_t *)s_stack + w * 7 * DR_WSTACK_LDS;
-    if (w & 1) tree_stack_run<7>(ops, seed, lds, out);
-    else tree_stack_run<5>(ops, seed, lds, out);
+    DR_LDS uint32_t *lds = (DR_LDS uint32_t *)s_stack + w * 6 * DR_WSTACK_LDS;
+    if (w & 1) tree_stack_run<6>(ops, seed, lds, out);
+    else tree_stack_run<4>(ops, seed, lds, out);
+}
+
+// dr_test_tree_walk: every wave walks 64 trees, one node a lane and iteration as
+// the selection kernel, whose every inner node has a leaf and below it, on top of
+// the stack, the rest of the tree: the shape that grows the stack by a whole wave's
+// entries per level.  An entry: id, levels below, and words made from them.
+// out: entries popped that differ, nodes visited, nodes lost at a full stack,
+// most entries held.
+template <int WORDS>
+DR_INLINE void tree_walk_run(int levels, bool throttle, DR_LDS uint32_t *lds, unsigned long long *out) {
+    const int lane = (int)__lane_id();
+    WaveStack<WORDS> A;
+    WaveSpill<WORDS> spill;
+    A.init(lds);
+    unsigned long long bad = 0, visited = 0, lost = 0;
+    int most = 0;
+    auto push = [&](bool have, uint32_t id, int below) {
+        uint32_t x[WORDS];
+        x[0] = id;
+        x[1] = (uint32_t)below;
+        for (int r = 2; r < WORDS; r++) x[r] = id * 0x9E3779B9u ^ (uint32_t)below << (4 * r);
+        if (!A.push(have, x, lane, spill) && have) lost += 2ull * below + 1;
+        most = max(most, A.size());
+    };
+    push(true, blockIdx.x * blockDim.x + threadIdx.x, levels);
+    while (A.size() > 0) {
+        uint32_t x[WORDS] = {};
+        const bool run = A.pop(!(throttle && A.throttled()) || lane == 0, x, lane, spill);
+        if (run) {
+            visited++;
+            for (int r = 2; r < WORDS; r++)
+                if (x[r] != (x[0] * 0x9E3779B9u ^ x[1] << (4 * r))) bad++;
+        }
+        const bool inner = run && x[1] > 0;
+        push(inner, x[0] * 5u + 1u, 0);
+        push(inner, x[0] * 7u + 3u, (int)x[1] - 1);
+    }
+    atomicAdd(&out[0], bad);
+    atomicAdd(&out[1], visited);
+    atomicAdd(&out[2], lost);
+    atomicMax(&out[3], (unsigned long long)most);
+}
+__global__ void __launch_bounds__(DR_BLOCK) k_tree_walk(int levels, int throttle, unsigned long long *out) {
+    __shared__ uint32_t s_stack[6 * DR_WSTACK_LDS * (DR_BLOCK / 64)];
+    const int w = threadIdx.x >> 6;
+    DR_LDS uint32_t *lds = (DR_LDS uint32_t *)s_stack + w * 6 * DR_WSTACK_LDS;
+    if (w & 1) tree_walk_run<6>(levels, throttle != 0, lds, out);
+    else tree_walk_run<4>(levels, throttle != 0, lds, out);
 }
 
 __global__ void __launch_bounds__(256) k_line_integral(long long n, uint64_t seed, double *out) {
@@ -3161,6 +3217,23 @@ dr_status dr_test_tree_stack(int64_t ops, uint64_t seed, int64_t *out, void *str
     out[0] = (int64_t)r[0];
     out[1] = (int64_t)r[1];
     return launch_check("k_tree_stack");
+}
+
+dr_status dr_test_tree_walk(int levels, int throttle, int64_t *out, void *stream) {
+    if (levels < 0 || levels > 4096 || !out) return fail(DR_ERROR_INVALID_ARGUMENT, "bad arguments");
+    hipStream_t hs = (hipStream_t)stream;
+    unsigned long long *dev = nullptr;
+    if (hipMalloc(&dev, 4 * sizeof(unsigned long long)) != hipSuccess)
+        return fail(DR_ERROR_OUT_OF_MEMORY, "hipMalloc");
+    k_fill<<<1, 64, 0, hs>>>((float *)dev, 8, 0.f);
+    k_tree_walk<<<8, DR_BLOCK, 0, hs>>>(levels, throttle, dev);
+    unsigned long long r[4];
+    hipError_t e = hipMemcpyAsync(r, dev, sizeof(r), hipMemcpyDeviceToHost, hs);
+    if (e == hipSuccess) e = hipStreamSynchronize(hs);
+    (void)hipFree(dev);
+    if (e != hipSuccess) return fail(DR_ERROR_DEVICE, hipGetErrorString(e));
+    for (int i = 0; i < 4; i++) out[i] = (int64_t)r[i];
+    return launch_check("k_tree_walk");
 }
 
 dr_status dr_test_line_integral(int64_t num_samples, uint64_t seed, double *out, void *stream) {

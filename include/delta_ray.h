@@ -540,13 +540,22 @@ dr_status dr_scene_set_stat_shapes(dr_scene *scene, const int *shape_ids, int n)
  * stream. */
 dr_status dr_test_line_integral(int64_t num_samples, uint64_t seed, double *out, void *stream);
 
-/* Check of the edge-tree traversal stack the selection kernel keeps in LDS
- * (top entries in LDS, older ones spilled to private memory): every GPU lane
- * runs `ops` random pushes and pops on it and on a plain array stack.  out
- * (host, 2 int64): pops that differ (0 expected), deepest stack reached.  No
- * reference counterpart (a self-check of this implementation).  Synchronises
- * the stream. */
+/* Check of the stack of edge-tree nodes that the lanes of a wave share in the
+ * selection kernel (the top in LDS, blocks below it in private memory): every
+ * wave runs `ops` pushes and pops of random sets of its lanes on it and on a
+ * plain array, with the entry sizes of the plain and the learned selection.  out
+ * (host, 2 int64): pops that differ (0 expected), deepest stack reached, in
+ * entries per lane.  No reference counterpart (a self-check of this
+ * implementation).  Synchronises the stream. */
 dr_status dr_test_tree_stack(int64_t ops, uint64_t seed, int64_t *out, void *stream);
+
+/* The same stack driven as the selection drives it: 64 trees a wave of `levels`
+ * inner nodes in a chain (at most 4096), 32 waves, each lane expanding one node
+ * at a time.  throttle != 0: with the kernel's rule that lane 0 works alone while
+ * the stack is nearly full; 0: without it.  out (host, 4 int64): pops that
+ * differ, nodes visited, nodes lost at a full stack, most entries held.
+ * Synchronises the stream. */
+dr_status dr_test_tree_walk(int levels, int throttle, int64_t *out, void *stream);
 
 /* ----------------------------------------------------------- scene files
  * Mitsuba ".serialized" meshes (reference load_serialized.cpp:1-277, a
