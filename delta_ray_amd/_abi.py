@@ -197,6 +197,7 @@ ENTRY_POINTS = [
     ("dr_mlp_train", ctypes.c_int, [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p,
                                     ctypes.c_int64, ctypes.c_int, ctypes.c_int, ctypes.c_float, ctypes.c_uint64,
                                     ctypes.POINTER(ctypes.c_float), ctypes.c_void_p]),
+    ("dr_test_batch_queue_limit", ctypes.c_int, [ctypes.c_void_p, ctypes.c_int64, ctypes.POINTER(ctypes.c_int64)]),
     ("dr_test_tree_walk", ctypes.c_int, [ctypes.c_int, ctypes.c_int, ctypes.POINTER(ctypes.c_int64),
                                          ctypes.c_void_p]),
     ("dr_test_tree_stack", ctypes.c_int, [ctypes.c_int64, ctypes.c_uint64, ctypes.POINTER(ctypes.c_int64),

@@ -1545,6 +1545,15 @@ struct Tuning {
     int select_refill = 64;  // 1-64: depth first, fetching at most that many points at a time; 0: breadth first
 };
 
+// Entries the edge queue may grow to (36 B each with their lists); a pass that
+// selects more is sampled in parts.  Positions in the queue are kept in 32-bit
+// words (EdgeEntry::list, Workspace::cont), so it must stay below 2^31.  The line
+// lies lower: the longest passes known to run well hold 45 M entries (the 512 x
+// 512 heightfield), and one of 365 M has ended in a device error whose cause was
+// not found.
+#define DR_QUEUE_MAX (1ll << 27)
+static_assert(DR_QUEUE_MAX < (1ll << 31), "queue positions are 32-bit");
+
 // Device working set of the pipeline, grown on demand, and the hipGraph of
 // the last captured job list.
 struct Workspace {
@@ -1555,11 +1564,12 @@ struct Workspace {
     long long slot_cap = 0;
     EdgeEntry *q = nullptr;
     float4 *entry_dp = nullptr;
-    // queue entries left for k_edge_shade, and before them
-    // the list of the pass's points (k_sel_points: at most one per slot, and
-    // the queue has at least an entry per slot)
+    // queue entries left for k_edge_shade, and before them the list of the
+    // pass's points (k_sel_points: at most one per slot): an element per queue
+    // entry, and at least one per slot
     int *cont = nullptr;
-    long long q_cap = 0;
+    long long q_cap = 0, cont_cap = 0;
+    long long q_limit = DR_QUEUE_MAX;
     // queue length, -, largest queue length, continuations, largest frontier
     // end, largest leaf-list end (breadth-first selection), points listed
     // (DR_CNT_POINTS); then the point list's work counters, the samples drawn
@@ -1578,6 +1588,7 @@ struct Workspace {
     hipStream_t cap_stream = nullptr;        // stream graphs are captured on
     hipGraphExec_t exec = nullptr;
     std::vector<unsigned long long> graph_key;
+    std::vector<unsigned long long> split_key;  // the plan last found to need passes in parts, which no graph holds
     unsigned long long epoch = 0;            // counts reallocations (a captured graph is stale after one)
 };
 
@@ -2009,6 +2020,7 @@ static dr_status ensure_workspace_(Workspace &w, const Plan &P);
 static bool has_edges(const Plan &P);
 static dr_status grow_frontier(Workspace &w, long long n);
 static dr_status grow_leaves(Workspace &w, long long n);
+static dr_status grow_queue(Workspace &w, long long n);
 static dr_status ensure_workspace(Workspace &w, const Plan &P) {
     unsigned long long e0 = g_alloc_epoch;
     dr_status st = ensure_workspace_(w, P);
@@ -2054,14 +2066,10 @@ static dr_status ensure_workspace_(Workspace &w, const Plan &P) {
     }
     // four queue entries per point slot (the heightfield at 2 bounces selects
     // about 3.5); a pass that selects more grows the queue
-    long long qn = P.max_slots * 4;
-    if (qn > w.q_cap) {
-        if (!grow((void **)&w.q, qn * sizeof(EdgeEntry)) || !grow((void **)&w.entry_dp, qn * sizeof(float4)) ||
-            !grow((void **)&w.cont, qn * sizeof(int))) {
-            w.q_cap = 0;
-            return fail(DR_ERROR_OUT_OF_MEMORY, "adjoint edge queue");
-        }
-        w.q_cap = qn;
+    long long qn = std::min(P.max_slots * 4, w.q_limit);
+    if (qn > w.q_cap || P.max_slots > w.cont_cap) {
+        dr_status st = grow_queue(w, std::max(qn, w.q_cap));
+        if (st != DR_OK) return st;
     }
     if ((int)P.jobs.size() > w.jobs_cap) {
         if (!grow((void **)&w.jobs, P.jobs.size() * sizeof(DrJob))) return fail(DR_ERROR_OUT_OF_MEMORY, "job table");
@@ -2096,35 +2104,31 @@ static dr_status grow_leaves(Workspace &w, long long n) {
 
 static dr_status grow_queue(Workspace &w, long long n) {
     w.epoch++;
+    const long long c = std::max(n, w.slot_cap);
     if (!grow((void **)&w.q, n * sizeof(EdgeEntry)) || !grow((void **)&w.entry_dp, n * sizeof(float4)) ||
-        !grow((void **)&w.cont, n * sizeof(int))) {
-        w.q_cap = 0;
+        !grow((void **)&w.cont, c * sizeof(int))) {
+        w.q_cap = w.cont_cap = 0;
         return fail(DR_ERROR_OUT_OF_MEMORY, "adjoint edge queue");
     }
     w.q_cap = n;
+    w.cont_cap = c;
     return DR_OK;
 }
 
 static long long g_select_blocks[2] = {0, 0}, g_trace_blocks = 0, g_draw_blocks = 0, g_shade_blocks[4] = {0, 0, 0, 0};
 static long long g_sel_blocks[3] = {0, 0, 0};
 
-// All launches of a plan, stream-ordered, without host synchronisation (so
-// they can be captured in a hipGraph).  The tables are already on the device.
-static dr_status grow_queue(Workspace &w, long long n);
-
-// After a pass's edge selection, when the host may wait (no graph capture):
-// read the queue length and, if the queue overflowed, grow it and run the
-// selection of that pass again (it only writes the queue and the per-point
-// counts, so a second run replaces the first).
 // Grows what overflowed (edge queue; breadth-first frontier and leaf list)
-// after the counters cnt[0..5] were read into w.cnt_host; grew: whether
-// something did.
-static dr_status grow_overflowed(Workspace &w, long long qlen, bool bfs, bool &grew) {
+// after the counters cnt[0..5] were read into w.cnt_host.  grew: whether
+// something did; split: whether the queue would pass its limit (it then has
+// that length).
+static dr_status grow_overflowed(Workspace &w, long long qlen, bool bfs, bool &grew, bool &split) {
     grew = false;
-    if (qlen > w.q_cap) {
-        dr_status st = grow_queue(w, qlen + qlen / 4);
+    split = qlen > std::max(w.q_cap, w.q_limit);
+    if (qlen > w.q_cap && w.q_cap < w.q_limit) {
+        dr_status st = grow_queue(w, std::min(qlen + qlen / 4, w.q_limit));
         if (st != DR_OK) return st;
-        grew = true;
+        grew = !split;
     }
     if (bfs) {
         long long f = (long long)w.cnt_host[4], l = (long long)w.cnt_host[5];
@@ -2177,23 +2181,82 @@ static void launch_edge_trace(const Workspace &w, hipStream_t hs) {
                                                                                               w.entry_dp, w.cont);
 }
 
+// After a pass's edge selection, when the host may wait (no graph capture):
+// read the queue length and, if the queue overflowed, grow it and run the
+// selection of that pass again (it only writes the queue and the per-point
+// counts, so a second run replaces the first).  split: the pass selects more
+// than the queue may hold; len: how many.
 template <class Launch>
-static dr_status settle_selection(Workspace &w, hipStream_t hs, bool bfs, Launch &&select) {
+static dr_status settle_selection(Workspace &w, hipStream_t hs, bool bfs, Launch &&select, bool &split, long long &len) {
     for (int attempt = 0; attempt < 8; attempt++) {
         if (hipMemcpyAsync(w.cnt_host, w.cnt, 6 * sizeof(unsigned long long), hipMemcpyDeviceToHost, hs) !=
                 hipSuccess ||
             hipStreamSynchronize(hs) != hipSuccess)
             return fail(DR_ERROR_DEVICE, "reading the edge queue length failed");
         bool grew = false;
-        dr_status st = grow_overflowed(w, (long long)w.cnt_host[0], bfs, grew);
-        if (st != DR_OK) return st;
-        if (!grew) return DR_OK;
+        len = (long long)w.cnt_host[0];
+        dr_status st = grow_overflowed(w, len, bfs, grew, split);
+        if (st != DR_OK || split || !grew) return st;
         k_fill<<<1, 64, 0, hs>>>((float *)w.cnt, 4, 0.f);
         select();
     }
     return fail(DR_ERROR_DEVICE, "edge queue kept overflowing");
 }
 
+// The edge samples of a pass's (or a part's) selected edges.
+template <int MAXB>
+static void launch_edges(const Workspace &w, const Pass &ps, Timing *tm, hipStream_t hs) {
+    {
+        LaunchTimer t(tm, TK_EDGE, hs);
+        launch_edge_trace(w, hs);
+    }
+    {
+        LaunchTimer t(tm, TK_SHADE, hs);
+        long long sb = resident_blocks(k_edge_shade<MAXB>,
+                                       g_shade_blocks[MAXB == 1 ? 0 : MAXB == 2 ? 1 : MAXB == 4 ? 2 : 3]);
+        k_edge_shade<MAXB><<<(unsigned)sb, DR_BLOCK, 0, hs>>>(w.jobs, w.q, w.cnt, w.pts, w.pt_dp, w.pt_lastj,
+                                                              w.entry_dp, w.cont);
+    }
+    if (ps.dp_last) k_dp_last<<<1024, DR_BLOCK, 0, hs>>>(w.q, w.cnt, w.q_cap, w.entry_dp, w.pt_lastj, w.pt_dp);
+}
+
+// Selects and samples a pass in parts whose edges fit the queue (a shading
+// point's edges always fall in one part, so its Dirac derivatives and the
+// last-ordinal rule see all of them).  per: selected edges per point slot, which
+// sizes the parts (negative: not known yet); updated.
+template <int MAXB>
+static dr_status run_parts(const Plan &P, Workspace &w, const Pass &ps, double &per, Timing *tm, hipStream_t hs) {
+    long long part = per > 0.0 ? std::max(1ll, (long long)(0.9 * (double)w.q_cap / per)) : ps.nslots;
+    for (long long f0 = 0; f0 < ps.nslots;) {
+        long long f1 = std::min(ps.nslots, f0 + part);
+        k_fill<<<1, 64, 0, hs>>>((float *)w.cnt, 2 * 2, 0.f);       // queue length
+        k_fill<<<1, 64, 0, hs>>>((float *)(w.cnt + 3), 2, 0.f);     // continuations
+        {
+            LaunchTimer t(tm, TK_SELECT, hs);
+            // (the depth-first selection: its working set has a fixed size)
+            launch_select(P, w, ps.nslots, MAXB, P.select_refill > 0 ? P.select_refill : 64, f0, f1, hs);
+        }
+        unsigned long long len = 0;
+        if (hipMemcpyAsync(&len, w.cnt, sizeof(len), hipMemcpyDeviceToHost, hs) != hipSuccess ||
+            hipStreamSynchronize(hs) != hipSuccess)
+            return fail(DR_ERROR_DEVICE, "reading the edge queue length failed");
+        per = (double)len / (double)(f1 - f0);
+        if ((long long)len > w.q_cap) {
+            if (f1 - f0 <= 1)
+                return fail(DR_ERROR_UNSUPPORTED, "a shading point selects more edges than the edge queue holds");
+            part = std::max(1ll, std::min((f1 - f0) / 2, (long long)(0.9 * (double)w.q_cap / per)));
+            continue;
+        }
+        launch_edges<MAXB>(w, ps, tm, hs);
+        f0 = f1;
+        if (per > 0.0) part = std::max(1ll, (long long)(0.9 * (double)w.q_cap / per));
+    }
+    return DR_OK;
+}
+
+// All launches of a plan, stream-ordered, without host synchronisation (so
+// they can be captured in a hipGraph) unless sync_select.  The tables are
+// already on the device.
 // sync_select: settle every pass's queue length on the host before its edge
 // samples (uncaptured runs); otherwise the caller checks the largest length
 // once at the end.
@@ -2202,7 +2265,6 @@ static dr_status enqueue(const Plan &P, Workspace &w, Timing *tm, hipStream_t hs
     for (auto &z : P.zero) k_fill<<<256, 256, 0, hs>>>(z.first, z.second, 0.f);
     k_fill<<<1, 64, 0, hs>>>((float *)(w.cnt + 2), 8, 0.f);  // largest queue, continuations, largest lists
     const bool bfs = P.select_refill == 0;
-    const int bi = MAXB == 1 ? 0 : MAXB == 2 ? 1 : MAXB == 4 ? 2 : 3;
     for (const Pass &ps : P.passes) {
         const DrRange *R = w.ranges + ps.r0;
         int nr = ps.r1 - ps.r0;
@@ -2235,21 +2297,17 @@ static dr_status enqueue(const Plan &P, Workspace &w, Timing *tm, hipStream_t hs
             }
         };
         select();
+        bool split = false;
         if (sync_select) {
-            dr_status st = settle_selection(w, hs, bfs, select);
+            long long len = 0;
+            dr_status st = settle_selection(w, hs, bfs, select, split, len);
+            if (st == DR_OK && split) {
+                double per = (double)len / (double)ps.nslots;
+                st = run_parts<MAXB>(P, w, ps, per, tm, hs);
+            }
             if (st != DR_OK) return st;
         }
-        {
-            LaunchTimer t(tm, TK_EDGE, hs);
-            launch_edge_trace(w, hs);
-        }
-        {
-            LaunchTimer t(tm, TK_SHADE, hs);
-            long long sb = resident_blocks(k_edge_shade<MAXB>, g_shade_blocks[bi]);
-            k_edge_shade<MAXB><<<(unsigned)sb, DR_BLOCK, 0, hs>>>(w.jobs, w.q, w.cnt, w.pts, w.pt_dp, w.pt_lastj,
-                                                                  w.entry_dp, w.cont);
-        }
-        if (ps.dp_last) k_dp_last<<<1024, DR_BLOCK, 0, hs>>>(w.q, w.cnt, w.q_cap, w.entry_dp, w.pt_lastj, w.pt_dp);
+        if (!split) launch_edges<MAXB>(w, ps, tm, hs);
         {
             LaunchTimer t(tm, TK_DP, hs);
             k_dp<MAXB><<<(unsigned)ps.nblocks, DR_BLOCK, 0, hs>>>(w.jobs, R, nr, w.pts, w.pt_dp, w.counts);
@@ -2286,10 +2344,11 @@ static bool has_edges(const Plan &P) {
 // launches are captured once and replayed as a hipGraph, and, when there are
 // secondary edges, the largest queue length is read once at the end; a queue
 // that overflowed is grown and the plan runs again (every output is
-// rewritten from zero by a run).
+// rewritten from zero by a run), uncaptured where a pass needs parts.
 static dr_status run_plan(const Plan &P, Workspace &w, Timing *tm, hipStream_t hs, bool use_graph) {
     dr_status st = ensure_workspace(w, P);
     if (st != DR_OK) return st;
+    if (use_graph && w.split_key == P.key) use_graph = false;
     for (int attempt = 0; attempt < 8; attempt++) {
         if (hipMemcpyAsync(w.jobs, P.jobs.data(), P.jobs.size() * sizeof(DrJob), hipMemcpyHostToDevice, hs) !=
                 hipSuccess ||
@@ -2336,14 +2395,23 @@ static dr_status run_plan(const Plan &P, Workspace &w, Timing *tm, hipStream_t h
         st = launch_check("render kernels");
         if (st != DR_OK) return st;
         if (!has_edges(P)) return DR_OK;
+        if (!use_graph) {  // (every pass was settled)
+            if (hipStreamSynchronize(hs) != hipSuccess) return fail(DR_ERROR_DEVICE, "the render kernels failed");
+            return DR_OK;
+        }
         if (hipMemcpyAsync(w.cnt_host, w.cnt, 6 * sizeof(unsigned long long), hipMemcpyDeviceToHost, hs) !=
                 hipSuccess ||
             hipStreamSynchronize(hs) != hipSuccess)
             return fail(DR_ERROR_DEVICE, "reading the edge queue length failed");
-        bool grew = false;
-        st = grow_overflowed(w, (long long)w.cnt_host[2], P.select_refill == 0, grew);
+        bool grew = false, split = false;
+        st = grow_overflowed(w, (long long)w.cnt_host[2], P.select_refill == 0, grew, split);
         if (st != DR_OK) return st;
-        if (!grew) return DR_OK;
+        if (split) {
+            w.split_key = P.key;
+            use_graph = false;
+        } else if (!grew) {
+            return DR_OK;
+        }
     }
     return fail(DR_ERROR_DEVICE, "edge queue kept overflowing");
 }
@@ -2369,9 +2437,7 @@ static dr_status single_job(dr_scene *s, const dr_render_options *o, const float
 // inputs and outputs in `scratch`, a fixed array of this library (each GPU
 // the library runs on holds its own copy until the process ends), for
 // callers that cannot allocate.  Its passes are sized to fit the array; a
-// pass whose edge selection overflows the queue part of it is selected and
-// sampled in parts (a shading point's edges always fall in one part, so its
-// Dirac derivatives and the last-ordinal rule see all of them).
+// pass whose edge selection overflows the queue part of it is run in parts.
 #define DR_NOALLOC_BYTES (256ull << 20)
 #define DR_NOALLOC_QUEUE_PER_SLOT 1
 #define DR_NOALLOC_MAX_RANGES 4096
@@ -2411,7 +2477,7 @@ template <int MAXB>
 static dr_status run_noalloc(const Plan &P, Workspace &w, hipStream_t hs) {
     for (auto &z : P.zero) k_fill<<<256, 256, 0, hs>>>(z.first, z.second, 0.f);
     k_fill<<<1, 64, 0, hs>>>((float *)(w.cnt + 2), 2, 0.f);
-    double per = -1.0;  // selected edges per point of the last part (sizes the next one)
+    double per = -1.0;
     for (const Pass &ps : P.passes) {
         const DrRange *R = w.ranges + ps.r0;
         int nr = ps.r1 - ps.r0;
@@ -2419,35 +2485,8 @@ static dr_status run_noalloc(const Plan &P, Workspace &w, hipStream_t hs) {
         if (!ps.edges) continue;
         k_fill<<<1024, 256, 0, hs>>>(w.pt_dp, (size_t)ps.nslots * 3, 0.f);
         k_fill_i<<<1024, 256, 0, hs>>>(w.pt_lastj, (size_t)ps.nslots, -1);
-        long long part = per > 0.0 ? std::max(1ll, (long long)(0.9 * (double)w.q_cap / per)) : ps.nslots;
-        for (long long f0 = 0; f0 < ps.nslots;) {
-            long long f1 = std::min(ps.nslots, f0 + part);
-            k_fill<<<1, 64, 0, hs>>>((float *)w.cnt, 2 * 2, 0.f);       // queue length
-            k_fill<<<1, 64, 0, hs>>>((float *)(w.cnt + 3), 2, 0.f);     // continuations
-            // (the depth-first selection: its working set fits the array)
-            launch_select(P, w, ps.nslots, MAXB, P.select_refill > 0 ? P.select_refill : 64, f0, f1, hs);
-            unsigned long long len = 0;
-            if (hipMemcpyAsync(&len, w.cnt, sizeof(len), hipMemcpyDeviceToHost, hs) != hipSuccess ||
-                hipStreamSynchronize(hs) != hipSuccess)
-                return fail(DR_ERROR_DEVICE, "reading the edge queue length failed");
-            per = (double)len / (double)(f1 - f0);
-            if ((long long)len > w.q_cap) {
-                if (f1 - f0 <= 1)
-                    return fail(DR_ERROR_UNSUPPORTED, "a shading point selects more edges than the allocation-free "
-                                                      "queue holds");
-                part = std::max(1ll, std::min((f1 - f0) / 2, (long long)(0.9 * (double)w.q_cap / per)));
-                continue;
-            }
-            launch_edge_trace(w, hs);
-            long long sb = resident_blocks(k_edge_shade<MAXB>,
-                                           g_shade_blocks[MAXB == 1 ? 0 : MAXB == 2 ? 1 : MAXB == 4 ? 2 : 3]);
-            k_edge_shade<MAXB><<<(unsigned)sb, DR_BLOCK, 0, hs>>>(w.jobs, w.q, w.cnt, w.pts, w.pt_dp, w.pt_lastj,
-                                                                  w.entry_dp, w.cont);
-            if (ps.dp_last)
-                k_dp_last<<<1024, DR_BLOCK, 0, hs>>>(w.q, w.cnt, w.q_cap, w.entry_dp, w.pt_lastj, w.pt_dp);
-            f0 = f1;
-            if (per > 0.0) part = std::max(1ll, (long long)(0.9 * (double)w.q_cap / per));
-        }
+        dr_status st = run_parts<MAXB>(P, w, ps, per, nullptr, hs);
+        if (st != DR_OK) return st;
         k_dp<MAXB><<<(unsigned)ps.nblocks, DR_BLOCK, 0, hs>>>(w.jobs, R, nr, w.pts, w.pt_dp, w.counts);
     }
     if (P.prim_r1 > P.prim_r0)
@@ -3217,6 +3256,14 @@ dr_status dr_test_tree_stack(int64_t ops, uint64_t seed, int64_t *out, void *str
     out[0] = (int64_t)r[0];
     out[1] = (int64_t)r[1];
     return launch_check("k_tree_stack");
+}
+
+dr_status dr_test_batch_queue_limit(dr_batch *b, int64_t entries, int64_t *before) {
+    if (!b || entries < 1 || entries > DR_QUEUE_MAX) return fail(DR_ERROR_INVALID_ARGUMENT, "bad queue limit");
+    if (before) *before = b->ws.q_limit;
+    b->ws.q_limit = entries;
+    b->ws.split_key.clear();
+    return DR_OK;
 }
 
 dr_status dr_test_tree_walk(int levels, int throttle, int64_t *out, void *stream) {

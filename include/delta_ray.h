@@ -549,6 +549,11 @@ dr_status dr_test_line_integral(int64_t num_samples, uint64_t seed, double *out,
  * implementation).  Synchronises the stream. */
 dr_status dr_test_tree_stack(int64_t ops, uint64_t seed, int64_t *out, void *stream);
 
+/* Lowers the number of selected edges that a pass of the batch holds at once
+ * (2^27; a pass that selects more is sampled in parts), for tests of the parts.
+ * before (or NULL): the former number. */
+dr_status dr_test_batch_queue_limit(dr_batch *batch, int64_t entries, int64_t *before);
+
 /* The same stack driven as the selection drives it: 64 trees a wave of `levels`
  * inner nodes in a chain (at most 4096), 32 waves, each lane expanding one node
  * at a time.  throttle != 0: with the kernel's rule that lane 0 works alone while
