@@ -1199,10 +1199,23 @@ __global__ void __launch_bounds__(DR_BLOCK) k_dp(const DrJob *__restrict__ jobs,
     gc_flush(gkey, gval, DR_GC_SLOTS_SMALL, [&](int j) { return jobs[j].grads; });
 }
 
-__global__ void k_fill_i(int *p, size_t n, int v) {
-    size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    size_t stride = (size_t)gridDim.x * blockDim.x;
-    for (; i < n; i += stride) p[i] = v;
+// The counters of one selection and its edge samples: queue length, continuations
+// and the lists' counters (not the largest lengths, cnt[2], cnt[4] and cnt[5]).
+DR_INLINE void clear_counters(unsigned long long *cnt) {
+    for (int i = threadIdx.x; i < DR_CNT_WORDS; i += blockDim.x)
+        if (i < 2 || i == 3 || i >= DR_CNT_POINTS) cnt[i] = 0;
+}
+__global__ void k_part_begin(unsigned long long *cnt) { clear_counters(cnt); }
+// The same, and the Dirac derivatives and last ordinals of a pass's points: one
+// launch, where a small render would wait for six.
+__global__ void __launch_bounds__(DR_BLOCK) k_pass_begin(unsigned long long *cnt, float *pt_dp, int *pt_lastj,
+                                                         long long nslots) {
+    if (blockIdx.x == 0) clear_counters(cnt);
+    const long long stride = (long long)gridDim.x * blockDim.x;
+    for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < 3 * nslots; i += stride) {
+        pt_dp[i] = 0.f;
+        if (i < nslots) pt_lastj[i] = -1;
+    }
 }
 
 // primary-edge samples; a range is a piece [t0, t1) of one job's samples
@@ -2148,6 +2161,11 @@ static dr_status grow_overflowed(Workspace &w, long long qlen, bool bfs, bool &g
     return DR_OK;
 }
 
+static void launch_pass_begin(const Workspace &w, const Pass &ps, hipStream_t hs) {
+    k_pass_begin<<<(unsigned)std::min<long long>(1024, grid_of(3 * ps.nslots)), DR_BLOCK, 0, hs>>>(w.cnt, w.pt_dp,
+                                                                                                   w.pt_lastj, ps.nslots);
+}
+
 // The depth-first selection of the points f in [f0, f1): one resident grid of
 // one-wave workgroups.  A wave fetches at least 4 slots at a time, more where
 // the trees are so small that no point's walk is long: fetches of 4 cost the
@@ -2162,7 +2180,6 @@ static void launch_select(const Plan &P, const Workspace &w, long long nslots, i
     int fetch_min = std::min(fetch_max, std::max(4, std::min(64, 4096 / std::max(1, P.tree_nodes))));
     unsigned grid = (unsigned)std::min<long long>(waves, (n + fetch_min - 1) / fetch_min);
     const int per_block = DR_BLOCK * DR_LIST_PER_THREAD;
-    k_fill<<<1, 256, 0, hs>>>((float *)(w.cnt + DR_CNT_POINTS), 2 * (DR_CNT_DRAWN - DR_CNT_POINTS), 0.f);
     k_sel_points<<<(unsigned)((n + per_block - 1) / per_block), DR_BLOCK, 0, hs>>>(nslots, maxb, w.pts, w.cont, w.cnt,
                                                                                   w.counts, f0, f1);
     if (P.learned)
@@ -2174,7 +2191,6 @@ static void launch_select(const Plan &P, const Workspace &w, long long nslots, i
 // The selected edges' samples up to their side rays (resident grids: the
 // queue's length is known on the device only).
 static void launch_edge_trace(const Workspace &w, hipStream_t hs) {
-    k_fill<<<1, 256, 0, hs>>>((float *)(w.cnt + DR_CNT_DRAWN), 2 * (DR_CNT_WORDS - DR_CNT_DRAWN), 0.f);
     k_edge_draw<<<(unsigned)resident_blocks(k_edge_draw, g_draw_blocks), DR_BLOCK, 0, hs>>>(w.jobs, w.q, w.cnt, w.q_cap,
                                                                                            w.pts, w.entry_dp);
     k_edge_trace<<<(unsigned)resident_blocks(k_edge_trace, g_trace_blocks), DR_BLOCK, 0, hs>>>(w.jobs, w.q, w.cnt, w.pts,
@@ -2197,7 +2213,7 @@ static dr_status settle_selection(Workspace &w, hipStream_t hs, bool bfs, Launch
         len = (long long)w.cnt_host[0];
         dr_status st = grow_overflowed(w, len, bfs, grew, split);
         if (st != DR_OK || split || !grew) return st;
-        k_fill<<<1, 64, 0, hs>>>((float *)w.cnt, 4, 0.f);
+        k_part_begin<<<1, 256, 0, hs>>>(w.cnt);
         select();
     }
     return fail(DR_ERROR_DEVICE, "edge queue kept overflowing");
@@ -2223,14 +2239,15 @@ static void launch_edges(const Workspace &w, const Pass &ps, Timing *tm, hipStre
 // Selects and samples a pass in parts whose edges fit the queue (a shading
 // point's edges always fall in one part, so its Dirac derivatives and the
 // last-ordinal rule see all of them).  per: selected edges per point slot, which
-// sizes the parts (negative: not known yet); updated.
+// sizes the parts (negative: not known yet); updated.  cleared: the counters are.
 template <int MAXB>
-static dr_status run_parts(const Plan &P, Workspace &w, const Pass &ps, double &per, Timing *tm, hipStream_t hs) {
+static dr_status run_parts(const Plan &P, Workspace &w, const Pass &ps, double &per, bool cleared, Timing *tm,
+                           hipStream_t hs) {
     long long part = per > 0.0 ? std::max(1ll, (long long)(0.9 * (double)w.q_cap / per)) : ps.nslots;
     for (long long f0 = 0; f0 < ps.nslots;) {
         long long f1 = std::min(ps.nslots, f0 + part);
-        k_fill<<<1, 64, 0, hs>>>((float *)w.cnt, 2 * 2, 0.f);       // queue length
-        k_fill<<<1, 64, 0, hs>>>((float *)(w.cnt + 3), 2, 0.f);     // continuations
+        if (!cleared) k_part_begin<<<1, 256, 0, hs>>>(w.cnt);
+        cleared = false;
         {
             LaunchTimer t(tm, TK_SELECT, hs);
             // (the depth-first selection: its working set has a fixed size)
@@ -2273,10 +2290,7 @@ static dr_status enqueue(const Plan &P, Workspace &w, Timing *tm, hipStream_t hs
             k_path<MAXB><<<(unsigned)ps.nblocks, DR_BLOCK, 0, hs>>>(w.jobs, R, nr, w.pts);
         }
         if (!ps.edges) continue;
-        k_fill<<<1024, 256, 0, hs>>>(w.pt_dp, (size_t)ps.nslots * 3, 0.f);
-        k_fill_i<<<1024, 256, 0, hs>>>(w.pt_lastj, (size_t)ps.nslots, -1);
-        k_fill<<<1, 64, 0, hs>>>((float *)w.cnt, 4, 0.f);        // queue length
-        k_fill<<<1, 64, 0, hs>>>((float *)(w.cnt + 3), 2, 0.f);  // continuations
+        launch_pass_begin(w, ps, hs);
         auto select = [&]() {
             LaunchTimer t(tm, TK_SELECT, hs);
             if (bfs) {
@@ -2303,7 +2317,7 @@ static dr_status enqueue(const Plan &P, Workspace &w, Timing *tm, hipStream_t hs
             dr_status st = settle_selection(w, hs, bfs, select, split, len);
             if (st == DR_OK && split) {
                 double per = (double)len / (double)ps.nslots;
-                st = run_parts<MAXB>(P, w, ps, per, tm, hs);
+                st = run_parts<MAXB>(P, w, ps, per, false, tm, hs);
             }
             if (st != DR_OK) return st;
         }
@@ -2483,9 +2497,8 @@ static dr_status run_noalloc(const Plan &P, Workspace &w, hipStream_t hs) {
         int nr = ps.r1 - ps.r0;
         k_path<MAXB><<<(unsigned)ps.nblocks, DR_BLOCK, 0, hs>>>(w.jobs, R, nr, w.pts);
         if (!ps.edges) continue;
-        k_fill<<<1024, 256, 0, hs>>>(w.pt_dp, (size_t)ps.nslots * 3, 0.f);
-        k_fill_i<<<1024, 256, 0, hs>>>(w.pt_lastj, (size_t)ps.nslots, -1);
-        dr_status st = run_parts<MAXB>(P, w, ps, per, nullptr, hs);
+        launch_pass_begin(w, ps, hs);
+        dr_status st = run_parts<MAXB>(P, w, ps, per, true, nullptr, hs);
         if (st != DR_OK) return st;
         k_dp<MAXB><<<(unsigned)ps.nblocks, DR_BLOCK, 0, hs>>>(w.jobs, R, nr, w.pts, w.pt_dp, w.counts);
     }
