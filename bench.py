@@ -45,7 +45,7 @@ METRIC = "fwd+adjoint samples/s; time to gradient rel-RMSE 1e-2, learned vs plai
 
 # algorithmic bytes: the records each unit of work must read or write once
 B_RAY_IO = 32 + 16      # ray in (org, dir, tmin, tmax) + hit out (ids, u, v)
-B_NODE = 64             # one BVH2 node (two child boxes)
+B_NODE = 32             # one packed BVH2 node (two child boxes)
 B_TRI = 48              # one triangle (v0, e1, e2)
 B_PIXEL_IO = 12 + 12    # d_image read + image write per pixel sample
 B_EDGE = 24 + 24 + 24 + 24 + 36  # edge v0/v1, faces, non-shared verts, normals, LTC matrix

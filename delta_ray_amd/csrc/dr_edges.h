@@ -357,7 +357,7 @@ struct TreeAlt {
 // nearly in use, throttled() asks the caller to let lane 0 alone pop, expand
 // and push: a depth-first walk adds at most one entry per tree level, for which
 // there is room beside two pushes of all lanes.  A push for which there is none
-// all the same writes nothing and returns false (counted, not silently dropped).
+// all the same writes nothing and is counted in `lost`.
 #define DR_WSTACK_LDS 128
 #define DR_WSTACK_BLOCKS 30
 #define DR_WSTACK_CAP (DR_WSTACK_BLOCKS * 64 + DR_WSTACK_LDS)  // 32 entries per lane
@@ -381,19 +381,23 @@ struct WaveStack {
     DR_LDS uint32_t *w;  // [WORDS][DR_WSTACK_LDS]
     int n, base;         // entries in LDS: ring positions base .. base + n - 1
     int blocks;          // blocks of 64 entries in the spill
+    int lost;            // entries that found the stack full
     DR_INLINE void init(DR_LDS uint32_t *lds) {
         w = lds;
-        n = base = blocks = 0;
+        n = base = blocks = lost = 0;
     }
     DR_INLINE int size() const { return n + 64 * blocks; }
     DR_INLINE bool throttled() const { return size() > DR_WSTACK_CAP - 2 * 64 - 40; }
     // lanes with `have` push their entry, lower lanes below higher ones
-    DR_INLINE bool push(bool have, const uint32_t *x, int lane, WaveSpill<WORDS> &spill) {
+    DR_INLINE void push(bool have, const uint32_t *x, int lane, WaveSpill<WORDS> &spill) {
         unsigned long long m = __ballot(have);
         int k = __popcll(m);
-        if (k == 0) return true;
+        if (k == 0) return;
         if (n + k > DR_WSTACK_LDS) {
-            if (blocks == DR_WSTACK_BLOCKS) return false;
+            if (blocks == DR_WSTACK_BLOCKS) {
+                lost += k;
+                return;
+            }
             int i = (base + lane) & (DR_WSTACK_LDS - 1);
             for (int r = 0; r < WORDS; r++) spill.w[blocks * WORDS + r] = w[r * DR_WSTACK_LDS + i];
             blocks++;
@@ -407,7 +411,6 @@ struct WaveStack {
         }
         n += k;
         wave_lds_fence();
-        return true;
     }
     // lanes with `want` take entries from the top, lower lanes first; true
     // for the lanes that got one
@@ -436,7 +439,6 @@ struct WaveStack {
 
 struct EdgeTraversal {
     const DrEdgeNode *nodes;
-    int num_nodes;
     bool directional;
     BoundCtx B;
     Cone cone;
@@ -474,9 +476,9 @@ DR_INLINE bool et_init(EdgeTraversal &T, Stack &stack, const DrSceneView &S, F3 
     // plain or learned root lengths)
     float pmf = 1.f, pmf_o = 1.f;
     if (!has_n) {
-        T.nodes = S.sil_nodes; T.num_nodes = S.num_sil_nodes; T.directional = false;
+        T.nodes = S.sil_nodes; T.directional = false;
     } else if (!has_s) {
-        T.nodes = S.nrm_nodes; T.num_nodes = S.num_nrm_nodes; T.directional = true;
+        T.nodes = S.nrm_nodes; T.directional = true;
     } else {
         float ni = S.nrm_nodes[0].total_length, si = S.sil_nodes[0].total_length;
         float npmf = ni / (ni + si), spmf = si / (ni + si);
@@ -496,11 +498,11 @@ DR_INLINE bool et_init(EdgeTraversal &T, Stack &stack, const DrSceneView &S, F3 
         }
         float u = philox_next(T.rc);
         if (u < npmf) {
-            T.nodes = S.nrm_nodes; T.num_nodes = S.num_nrm_nodes; T.directional = true;
+            T.nodes = S.nrm_nodes; T.directional = true;
             pmf = npmf;
             pmf_o = npmf_o;
         } else {
-            T.nodes = S.sil_nodes; T.num_nodes = S.num_sil_nodes; T.directional = false;
+            T.nodes = S.sil_nodes; T.directional = false;
             pmf = spmf;
             pmf_o = spmf_o;
         }
@@ -565,12 +567,6 @@ DR_INLINE int et_expand(EdgeTraversal &T, const TreeEntry &e, TreeAlt ea, const 
     const int ni = e.node(), mask = CONE ? e.mask() : e.mask() & 2;
     const float cone_pmf = CONE ? e.cone_pmf() : 0.f, all_pmf = e.all_pmf();
     int li = ni + 1, ri = e.off;
-    // (a child lies behind its parent, so every walk ends: the check only guards
-    // against a malformed tree)
-    if (ri <= li || ri >= T.num_nodes) {
-        if (S.stats) atomicAdd(&S.stats[7], 1ull);
-        return 0;
-    }
     const DrEdgeNode L = gptr(T.nodes)[li], R = gptr(T.nodes)[ri];
     bool all_split = e.split_all();
     bool lcs = true, rcs = true;

@@ -214,7 +214,6 @@ DR_INLINE void sel_ctx(const SelPoint &P, const DrJob &J, EdgeTraversal &T, SPoi
     const DrSceneView &S = J.S;
     bool nrm = (P.info & 1) != 0;
     T.nodes = nrm ? S.nrm_nodes : S.sil_nodes;
-    T.num_nodes = nrm ? S.num_nrm_nodes : S.num_sil_nodes;
     T.directional = nrm;
     T.B = P.B;
     T.cone = Cone{P.pos, P.cdir, P.ccos};
@@ -568,7 +567,6 @@ k_select(const DrJob *__restrict__ jobs, const int *list, const PointRec *pts, E
         uint32_t info = C[26 * 64 + pt];
         bool nrm = (info & 1) != 0;
         T.nodes = nrm ? J.S.nrm_nodes : J.S.sil_nodes;
-        T.num_nodes = nrm ? J.S.num_nrm_nodes : J.S.num_sil_nodes;
         T.directional = nrm;
         T.mode = LEARNED ? (int)(info >> 1) & 3 : 0;
         T.cone_pmf_quirk = (J.c.flags & DR_QUIRK_CONE_PMF) != 0;
@@ -679,16 +677,6 @@ k_select(const DrJob *__restrict__ jobs, const int *list, const PointRec *pts, E
         if (LEARNED) a = TreeAlt{__uint_as_float(x[SW - 2]), __uint_as_float(x[SW - 1])};
         return (x[0] >> 31) << 5 | (x[2] >> 31) << 4 | x[3] >> 28;
     };
-    // throttled() keeps room for every push; a stack that is full all the same
-    // would be counted, not silently dropped
-    auto push = [&](WaveStack<SW> &st, WaveSpill<SW> &spill, bool v, const uint32_t *x, uint32_t pt) {
-        if (st.push(v, x, lane, spill)) return;
-        int d0 = 0, d1 = 0;
-        half_count(v, pt, d0, d1);
-        out0 -= d0;
-        out1 -= d1;
-        if (jobs[job].S.stats && lane == 0) atomicAdd(&jobs[job].S.stats[7], (unsigned long long)(d0 + d1));
-    };
     // Fetches points until one is pending or none are left, then starts
     // pending points of one job.  False when nothing could be started now.
     auto start = [&]() -> bool {
@@ -761,7 +749,7 @@ k_select(const DrJob *__restrict__ jobs, const int *list, const PointRec *pts, E
         add_leaf(lf, rs.e, rs.a, pt);
         uint32_t x[SW];
         pack(x, rs.e, rs.a, pt);
-        push(cst, cspill, root && !lf, x, pt);
+        cst.push(root && !lf, x, lane, cspill);
         return true;
     };
 
@@ -799,8 +787,8 @@ k_select(const DrJob *__restrict__ jobs, const int *list, const PointRec *pts, E
             const bool leaf = v && c.nprims() > 0;
             const bool nc = CONE && et_need_cone(c, a);
             pack(x, c, a, pt);
-            if (CONE) push(cst, cspill, v && !leaf && nc, x, pt);
-            push(ast, aspill, v && !leaf && !nc, x, pt);
+            if (CONE) cst.push(v && !leaf && nc, x, lane, cspill);
+            ast.push(v && !leaf && !nc, x, lane, aspill);
             add_leaf(leaf, c, a, pt);
         };
         put(v0, c0, a0);
@@ -830,6 +818,10 @@ k_select(const DrJob *__restrict__ jobs, const int *list, const PointRec *pts, E
         if (ta || (!tc && (na >= 64 || (nc < 64 && na >= nc)))) expand(std::false_type(), ast, aspill, on);
         else expand(std::true_type(), cst, cspill, on);
     }
+    // throttled() keeps room for every push; a stack that was full all the same
+    // is counted, not silently dropped
+    if (cst.lost + ast.lost > 0 && jobs[job].S.stats && lane == 0)
+        atomicAdd(&jobs[job].S.stats[7], (unsigned long long)(cst.lost + ast.lost));
 }
 
 // C: edge samples.  Only about one in five passes the connectivity test of its
@@ -1393,7 +1385,9 @@ DR_INLINE void tree_walk_run(int levels, bool throttle, DR_LDS uint32_t *lds, un
         x[0] = id;
         x[1] = (uint32_t)below;
         for (int r = 2; r < WORDS; r++) x[r] = id * 0x9E3779B9u ^ (uint32_t)below << (4 * r);
-        if (!A.push(have, x, lane, spill) && have) lost += 2ull * below + 1;
+        const int before = A.lost;
+        A.push(have, x, lane, spill);
+        if (have && A.lost > before) lost += 2ull * below + 1;
         most = max(most, A.size());
     };
     push(true, blockIdx.x * blockDim.x + threadIdx.x, levels);

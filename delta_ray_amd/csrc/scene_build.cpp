@@ -752,6 +752,22 @@ bool bvh_in_order(const std::vector<DrNode> &nodes) {
     return true;
 }
 
+// An edge tree as its walks assume it: children behind their parent, so that
+// every walk ends, and every edge in one leaf.
+static bool edge_tree_in_order(const std::vector<DrEdgeNode> &nodes, size_t num_edges) {
+    size_t edges = 0;
+    for (size_t i = 0; i < nodes.size(); i++) {
+        const DrEdgeNode &n = nodes[i];
+        if (n.nprims > 0) {
+            if ((size_t)n.offset != edges) return false;
+            edges += n.nprims;
+        } else if (n.offset <= (int)i + 1 || n.offset >= (int)nodes.size()) {
+            return false;
+        }
+    }
+    return edges == num_edges;
+}
+
 std::string adopt_device_bvh(HostScene &hs, const std::vector<DrNode> &built, std::vector<DrTri> &tris) {
     int m = (int)built.size();
     if (m == 0) return "empty device BVH";
@@ -848,6 +864,8 @@ std::string build_structures(HostScene &hs) {
     // the ray traversal stack holds at most one far child per interior level
     if (hs.bvh_depth > DR_STACK) return "triangle BVH deeper than the traversal stack";
     if (!bvh_in_order(hs.nodes)) return "triangle BVH is not in depth-first order";
+    if (!edge_tree_in_order(hs.sil_nodes, hs.sil_edges.size()) || !edge_tree_in_order(hs.nrm_nodes, hs.nrm_edges.size()))
+        return "edge tree is not in depth-first order";
     build_geo_records(hs);
     // refit tables: levels of the three trees, edge ranges of the edge-tree nodes
     tree_levels((int)hs.nodes.size(), [&](int i, int *c) {
