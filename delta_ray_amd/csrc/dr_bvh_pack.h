@@ -5,22 +5,24 @@
 #include "dr_types.h"
 
 // One axis of a node's frame: planes at origin + q * step, q = 0 .. 255, the step
-// as the exponent bits of a float.
-// The step is the least power of two of which 252 span both boxes, and at least
-// two units in the last place of the largest coordinate, so that the origin,
-// one step below the boxes, rounds by at most half a step.  An axis with
-// coordinates that are not finite, or too large for sums of them, has the origin
-// not-a-number: so are all of its distances, and it does not constrain a ray.
+// (2^k or 1.5 * 2^k) as the top 9 bits of a float below its sign.  The step is the
+// least of which 253 span both boxes, and at least two units in the last place of
+// the largest coordinate; the origin lies a 32nd of a step below the boxes, or two
+// such units, so that it is a 64th of a step below them when rounded.  An axis
+// with coordinates that are not finite, or too large for sums of them, has the
+// origin not-a-number: so are all of its distances, and it does not constrain a ray.
 struct PackAxis {
     float origin, rstep;
-    uint32_t exponent;
+    uint32_t step;
 };
 DR_INLINE PackAxis pack_axis(float lo, float hi) {
     float most = fmaxf(fabsf(lo), fabsf(hi)), ext = hi - lo;
-    if (!(lo <= hi && most < 1e36f)) return PackAxis{__uint_as_float(0x7fc00000u), 0.f, 127u};
-    uint32_t b = __float_as_uint(fmaxf(fmaxf(ext * (1.f / 252.f), most * 2.384185791015625e-7f), 1e-30f));
-    uint32_t e = (b >> 23) + ((b & 0x7fffffu) != 0);
-    return PackAxis{lo - __uint_as_float(e << 23), __uint_as_float((254u - e) << 23), e};
+    if (!(lo <= hi && most < 1e36f)) return PackAxis{__uint_as_float(0x7fc00000u), 0.f, 127u << 1};
+    const float ulps = most * 2.384185791015625e-7f;
+    uint32_t b = __float_as_uint(fmaxf(fmaxf(ext * (1.f / 253.f), ulps), 1e-30f));
+    b = (b >> 22) + ((b & 0x3fffffu) != 0);
+    const float step = __uint_as_float(b << 22);
+    return PackAxis{lo - fmaxf(step * 0.03125f, ulps), 1.f / step, b};
 }
 // a lower / upper plane on the axis, at least a 64th of a step outside v: the
 // walk's rounding is at most 1e-4 of a step near the box (not-a-number: any)
@@ -40,7 +42,7 @@ DR_INLINE DrPackedNode pack_node(const DrNode &n, int i) {
     const bool none = !leaf1 && n.d[1] == 0;
     const bool swap = leaf0 && !leaf1 && !none;
     DrPackedNode p;
-    uint32_t exps = 0;
+    uint32_t steps = 0;
     auto boxes = [&](int k, float l0, float h0, float l1, float h1) {
         if (none) {
             l1 = l0;
@@ -51,13 +53,13 @@ DR_INLINE DrPackedNode pack_node(const DrNode &n, int i) {
         const uint32_t c0 = pack_lo(l0, a) | pack_hi(h0, a) << 8, c1 = pack_lo(l1, a) | pack_hi(h1, a) << 8;
         p.w[k] = __float_as_uint(a.origin);
         p.w[4 + k] = swap ? c1 | c0 << 16 : c0 | c1 << 16;
-        exps |= a.exponent << (23 - 8 * k);
+        steps |= a.step << (22 - 9 * k);
     };
     boxes(0, n.a[0], n.a[3], n.b[2], n.c[1]);
     boxes(1, n.a[1], n.b[0], n.b[3], n.c[2]);
     boxes(2, n.a[2], n.b[1], n.c[0], n.c[3]);
     const uint32_t n0 = leaf0 && !swap ? (uint32_t)n.d[2] : 0u, n1 = leaf1 ? (uint32_t)n.d[3] : (swap ? (uint32_t)n.d[2] : 0u);
-    p.w[3] = exps | (n0 > 0 ? 0x80000000u : 0u) | (leaf0 || leaf1 ? 1u : 0u) | n0 << 1 | n1 << 3;
+    p.w[3] = steps | (leaf0 || leaf1 ? 0x80000000u : 0u) | n0 | n1 << 2;
     p.w[7] = (uint32_t)(leaf0 ? n.d[0] : n.d[1]);
     return p;
 }

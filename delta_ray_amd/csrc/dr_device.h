@@ -67,12 +67,12 @@ struct NodeFetch {
         Q = n[1];
         next = node + 1;
     }
-    DR_INLINE bool leaf(int c) const { return c == 0 ? (int)P.w < 0 : (P.w & 1u) != 0; }
+    DR_INLINE bool leaf(int c) const { return c == 0 ? (P.w & 3u) != 0 : (int)P.w < 0; }
     // the child's node
     DR_INLINE int child(int c) const { return c == 0 ? next : (int)Q.w; }
     // the triangles of the leaves among the children that are on: slots first .. end - 1
     DR_INLINE void leaves(bool on0, bool on1, int &first, int &end) const {
-        const uint32_t n0 = (P.w >> 1) & 3u, n1 = (P.w >> 3) & 3u;
+        const uint32_t n0 = P.w & 3u, n1 = (P.w >> 2) & 3u;
         first = (int)(Q.w + (on0 ? 0u : n0));
         end = (int)(Q.w + n0 + (on1 ? n1 : 0u));
     }
@@ -81,8 +81,8 @@ struct NodeFetch {
 struct FrameRay {
     F3 step, org;
     DR_INLINE FrameRay(const NodeFetch &N, F3 o, F3 inv) {
-        auto power = [&](int k) { return __uint_as_float((N.P.w << (8 * k)) & 0x7f800000u); };
-        step = F3{power(0) * inv.x, power(1) * inv.y, power(2) * inv.z};
+        auto len = [&](int k) { return __uint_as_float((N.P.w << (9 * k)) & 0x7fc00000u); };
+        step = F3{len(0) * inv.x, len(1) * inv.y, len(2) * inv.z};
         org = F3{(__uint_as_float(N.P.x) - o.x) * inv.x, (__uint_as_float(N.P.y) - o.y) * inv.y,
                  (__uint_as_float(N.P.z) - o.z) * inv.z};
     }

@@ -41,10 +41,11 @@ struct DrNode {
 // frame of the node's own (dr_bvh_pack.h), so that a box is wider than the
 // exact one by at most about a hundredth of its parent's at any scale of the
 // scene; half the bytes of a DrNode.  w[0..2]: the frame's origin; w[3]: its
-// steps' exponents (x in bits 23-30, y 15-22, z 7-14), bit 31 / 0: child 0 / 1 is
-// a leaf, bits 1-2 / 3-4: triangles of leaf 0 / 1 (0: not a leaf); w[4..6]: per
-// axis lo and hi of child 0, then of child 1; w[7]: the first triangle slot of
-// the leaves, or child 1's node.  Child 0's node is the next one.
+// steps (the top 9 bits of a float below its sign: x in bits 22-30, y 13-21, z
+// 4-12), bits 0-1 / 2-3: triangles of leaf 0 / 1 (0: not a leaf), bit 31: child 1
+// is a leaf; w[4..6]: per axis lo and hi of child 0, then of child 1; w[7]: the
+// first triangle slot of the leaves, or child 1's node.  Child 0's node is the
+// next one.
 struct alignas(16) DrPackedNode {
     uint32_t w[8];
 };
