@@ -47,13 +47,14 @@ DR_INLINE bool tri_hit(const DrTri &T, F3 org, F3 dir, float tmin, float tmax, f
     return u >= 0.f && v >= 0.f && u + v <= 1.f && t > tmin && t < tmax;
 }
 
-// 1 / direction of a ray, for box tests.  An axis the ray does not move along
-// (1 / dir infinite) does not constrain the interval: its factor is
-// not-a-number, which minima and maxima over the axes pass over.
+// 1 / direction of a ray, for box tests.  An axis the ray hardly moves along (1 /
+// dir infinite, or so large that a step's distance could be) does not constrain the
+// interval: its factor is not-a-number, which minima and maxima over the axes pass
+// over.
 DR_INLINE F3 box_inv(F3 dir) {
     auto rcp = [](float d) {
         float i = 1.f / d;
-        return fabsf(i) == DR_INF ? __uint_as_float(0x7fc00000u) : i;
+        return fabsf(i) < 1e18f ? i : __uint_as_float(0x7fc00000u);
     };
     return F3{rcp(dir.x), rcp(dir.y), rcp(dir.z)};
 }
@@ -77,45 +78,50 @@ struct NodeFetch {
         end = (int)(Q.w + n0 + (on1 ? n1 : 0u));
     }
 };
-// A ray's distances to the planes of a node's frame: t = q * step + org.
+// A ray's distances to the planes of a node's frame: t = q * step + org, of far
+// planes q * step + far.
 struct FrameRay {
-    F3 step, org;
+    F3 step, org, far;
     DR_INLINE FrameRay(const NodeFetch &N, F3 o, F3 inv) {
-        auto len = [&](int k) { return __uint_as_float((N.P.w << (9 * k)) & 0x7fc00000u); };
-        step = F3{len(0) * inv.x, len(1) * inv.y, len(2) * inv.z};
+        auto len = [&](int k, uint32_t o) { return __uint_as_float(((N.P.w << (9 * k)) & 0x7fc00000u) | o << 31); };
+        step = F3{len(0, N.P.x) * inv.x, len(1, N.P.y) * inv.y, len(2, N.P.z) * inv.z};
         org = F3{(__uint_as_float(N.P.x) - o.x) * inv.x, (__uint_as_float(N.P.y) - o.y) * inv.y,
                  (__uint_as_float(N.P.z) - o.z) * inv.z};
+        far = F3{fmaf(step.x, DR_PACK_FAR, org.x), fmaf(step.y, DR_PACK_FAR, org.y), fmaf(step.z, DR_PACK_FAR, org.z)};
     }
 };
-// Slab test of child c's box, widened by a relative 1e-5 (+1e-7) so that
-// rounding can never hide a triangle the exact test would accept: the planes
-// lie at least a 64th of a step outside the exact box.  Within 512 steps of the
-// frame the rounding of the distances is below 1e-4 of a step, and beyond it
-// below 5e-7 of the distance.  The widening is monotone, so the entry and exit
-// are widened once, after the max / min over the axes.
+// Slab test of child c's box, widened so that rounding can never hide a triangle
+// the exact test would accept: the planes lie at least a 4096th of a step outside
+// the exact box, the exit is raised by a relative 2e-5 (+2e-7) and the largest
+// distance by 1e-5 (+1e-7, box_limit), once per hit.  Within 512 steps of the frame the
+// rounding of the distances is below 1e-4 of a step, and beyond it below 5e-7 of
+// the distance.  The widening is monotone, so the exit is widened once, after the
+// minimum over the axes.
 //
-// Ray walks are bound by the latency and bytes of their node loads (16-byte
-// loads, a cache line per lane): with 32-byte nodes instead of 64-byte ones,
-// and sibling leaves' triangles in one loop, two at a time, a forward render of
-// the 32 k triangle heightfield (16.8 M samples) takes 6.8 ms instead of 8.6 and
-// a million plain rays 212 us instead of 334 (one at a time with the next one's
-// load ahead: single triangle adjoint 520 us instead of 510, shadow scene's 4.87
-// ms instead of 4.85).  Planes on one grid over the
-// whole scene would be simpler and as fast on these scenes, but a ground quad
-// 1000 times a mesh's size makes its rays visit twice the nodes, and one 100 000
-// times its size 600 times.
-DR_INLINE bool box_hit(const NodeFetch &N, int c, const FrameRay &f, float tmin, float tmax, float &tenter) {
-    auto lo = [&](uint32_t w) { return (float)(c ? (w >> 16) & 0xffu : w & 0xffu); };
-    auto hi = [&](uint32_t w) { return (float)(c ? w >> 24 : (w >> 8) & 0xffu); };
-    float ax = fmaf(lo(N.Q.x), f.step.x, f.org.x), bx = fmaf(hi(N.Q.x), f.step.x, f.org.x);
-    float ay = fmaf(lo(N.Q.y), f.step.y, f.org.y), by = fmaf(hi(N.Q.y), f.step.y, f.org.y);
-    float az = fmaf(lo(N.Q.z), f.step.z, f.org.z), bz = fmaf(hi(N.Q.z), f.step.z, f.org.z);
+// Ray walks are bound by the latency and bytes of their node loads (16-byte loads, a
+// cache line per lane) and by the vector work of the tests.  With 32-byte nodes
+// instead of 64-byte ones, and sibling leaves' triangles in one loop whose loads go
+// two at a time, a forward render of the 32 k triangle heightfield (16.8 M samples)
+// takes 6.8 ms instead of 8.6 and a million plain rays 212 us instead of 334.  Boxes a
+// step thick at both ends of a frame would have every ray that leaves a floor test the
+// floor's triangles again (a 200 x 150 forward render of the shadow scene 81 us
+// instead of 74).
+// Planes on one grid over the whole scene would be as fast on these scenes, but
+// beside a ground quad 500 times a 128 x 128 heightfield's size a ray visits 21 nodes
+// and 8 triangles instead of 16 and 3, and beside one 50 000 times its size 6 900 and
+// 13 000.
+DR_INLINE float box_limit(float tmax) { return fmaf(fabsf(tmax), 1e-5f, tmax) + 1e-7f; }
+DR_INLINE bool box_hit(const NodeFetch &N, int c, const FrameRay &f, float tmin, float limit, float &tenter) {
+    auto q0 = [&](uint32_t w) { return (float)(c ? (w >> 16) & 0xffu : w & 0xffu); };
+    auto q1 = [&](uint32_t w) { return (float)(c ? w >> 24 : (w >> 8) & 0xffu); };
+    float ax = fmaf(q0(N.Q.x), f.step.x, f.org.x), bx = fmaf(q1(N.Q.x), f.step.x, f.far.x);
+    float ay = fmaf(q0(N.Q.y), f.step.y, f.org.y), by = fmaf(q1(N.Q.y), f.step.y, f.far.y);
+    float az = fmaf(q0(N.Q.z), f.step.z, f.org.z), bz = fmaf(q1(N.Q.z), f.step.z, f.far.z);
     float mn = fmaxf(fmaxf(fminf(ax, bx), fminf(ay, by)), fminf(az, bz));
     float mx = fminf(fminf(fmaxf(ax, bx), fmaxf(ay, by)), fmaxf(az, bz));
-    mn = fmaf(fabsf(mn), -1e-5f, mn) - 1e-7f;
-    mx = fmaf(fabsf(mx), 1e-5f, mx) + 1e-7f;
+    mx = fmaf(fabsf(mx), 2e-5f, mx) + 2e-7f;
     tenter = fmaxf(mn, tmin);
-    return tenter <= fminf(mx, tmax);
+    return tenter <= fminf(mx, limit);
 }
 
 // Optional counters (rays, nodes visited, triangles tested) for the roofline
@@ -163,7 +169,7 @@ DR_INLINE Isect trace_closest(const DrSceneView &S, F3 org, F3 dir, float tmin, 
     Isect best = no_hit();
     if (S.num_nodes == 0) return best;
     const F3 inv = box_inv(dir);
-    float best_t = tmax;
+    float best_t = tmax, limit = box_limit(tmax);
     int best_g = -1;
     float bu = 0.f, bv = 0.f;
     TraceStack stack;
@@ -178,30 +184,30 @@ DR_INLINE Isect trace_closest(const DrSceneView &S, F3 org, F3 dir, float tmin, 
         nn++;
         const FrameRay f(N, org, inv);
         float t0, t1;
-        bool h0 = box_hit(N, 0, f, tmin, best_t, t0);
-        bool h1 = box_hit(N, 1, f, tmin, best_t, t1);
+        bool h0 = box_hit(N, 0, f, tmin, limit, t0);
+        bool h1 = box_hit(N, 1, f, tmin, limit, t1);
         // leaves first (the first child is a leaf only if both are)
         if ((h0 && N.leaf(0)) || (h1 && N.leaf(1))) {
             int i, end;
             N.leaves(h0 && N.leaf(0), h1, i, end);
-            // (two at a time, so that their loads and divisions overlap; a single one
-            // is tested twice, which changes nothing)
+            // (two at a time, so that their loads overlap; the array has one to spare)
+            auto test = [&](const DrTri &T) {
+                float u, v, t;
+                nt++;
+                if (tri_hit(T, org, dir, tmin, tmax, u, v, t)) {
+                    int g = __float_as_int(T.v0[3]);
+                    if (best_g < 0 || t < best_t || (t == best_t && g < best_g)) {
+                        best_t = t; best_g = g; bu = u; bv = v;
+                        limit = box_limit(t);
+                    }
+                }
+            };
             for (; i < end; i += 2) {
-                const DrTri T0 = gptr(S.tris)[i], T1 = gptr(S.tris)[min(i + 1, end - 1)];
-                float u, v, t, u1, v1, t1;
-                nt += i + 1 < end ? 2 : 1;
-                const bool hit0 = tri_hit(T0, org, dir, tmin, tmax, u, v, t);
-                const bool hit1 = tri_hit(T1, org, dir, tmin, tmax, u1, v1, t1);
-                int g = __float_as_int(T0.v0[3]);
-                if (hit0 && (best_g < 0 || t < best_t || (t == best_t && g < best_g))) {
-                    best_t = t; best_g = g; bu = u; bv = v;
-                }
-                g = __float_as_int(T1.v0[3]);
-                if (hit1 && (best_g < 0 || t1 < best_t || (t1 == best_t && g < best_g))) {
-                    best_t = t1; best_g = g; bu = u1; bv = v1;
-                }
+                const DrTri T0 = gptr(S.tris)[i], T1 = gptr(S.tris)[i + 1];
+                test(T0);
+                if (i + 1 < end) test(T1);
             }
-            h0 = h0 && !N.leaf(0) && t0 <= best_t;
+            h0 = h0 && !N.leaf(0) && t0 <= limit;
             h1 = false;
         }
         if (h0 && h1) {
@@ -246,6 +252,7 @@ struct Walk2 {
     F3 org, da, db;
     F3 ia, ib;     // 1 / da, 1 / db (box_inv)
     float ta, tb;  // closest distances so far
+    float la, lb;  // their box_limit
     int ga, gb;    // their triangles (global ids, -1: none)
     int node, sp;
     uint32_t nn, nt;
@@ -261,7 +268,7 @@ struct Walk2 {
         }
         ia = box_inv(da);
         ib = box_inv(db);
-        ta = tb = DR_INF;
+        ta = tb = la = lb = DR_INF;
         ga = gb = -1;
         node = sp = 0;
         nn = nt = 0;
@@ -274,10 +281,10 @@ struct Walk2 {
         nn++;
         const FrameRay fa(N, org, ia), fb(N, org, ib);
         float a0, a1, b0, b1;
-        bool ha0 = box_hit(N, 0, fa, tmin, ta, a0);
-        bool ha1 = box_hit(N, 1, fa, tmin, ta, a1);
-        bool hb0 = box_hit(N, 0, fb, tmin, tb, b0);
-        bool hb1 = box_hit(N, 1, fb, tmin, tb, b1);
+        bool ha0 = box_hit(N, 0, fa, tmin, la, a0);
+        bool ha1 = box_hit(N, 1, fa, tmin, la, a1);
+        bool hb0 = box_hit(N, 0, fb, tmin, lb, b0);
+        bool hb1 = box_hit(N, 1, fb, tmin, lb, b1);
         bool h0 = ha0 || hb0, h1 = ha1 || hb1;
         // leaves first (the first child is a leaf only if both are)
         if ((h0 && N.leaf(0)) || (h1 && N.leaf(1))) {
@@ -290,13 +297,15 @@ struct Walk2 {
                 nt++;
                 if (tri_hit(T, org, da, tmin, DR_INF, u, v, t) && (ga < 0 || t < ta || (t == ta && g < ga))) {
                     ta = t; ga = g;
+                    la = box_limit(t);
                 }
                 if (tri_hit(T, org, db, tmin, DR_INF, u, v, t) && (gb < 0 || t < tb || (t == tb && g < gb))) {
                     tb = t; gb = g;
+                    lb = box_limit(t);
                 }
             }
-            ha0 = ha0 && a0 <= ta;
-            hb0 = hb0 && b0 <= tb;
+            ha0 = ha0 && a0 <= la;
+            hb0 = hb0 && b0 <= lb;
             h0 = !N.leaf(0) && (ha0 || hb0);
             h1 = false;
         }
@@ -333,6 +342,7 @@ struct Walk2 {
 
 DR_INLINE bool trace_any(const DrSceneView &S, F3 org, F3 dir, float tmin, float tmax) {
     if (S.num_nodes == 0) return false;
+    const float limit = box_limit(tmax);
     const F3 inv = box_inv(dir);
     TraceStack stack;
     int sp = 0;
@@ -345,18 +355,20 @@ DR_INLINE bool trace_any(const DrSceneView &S, F3 org, F3 dir, float tmin, float
         nn++;
         const FrameRay f(N, org, inv);
         float t0, t1;
-        bool h0 = box_hit(N, 0, f, tmin, tmax, t0);
-        bool h1 = box_hit(N, 1, f, tmin, tmax, t1);
+        bool h0 = box_hit(N, 0, f, tmin, limit, t0);
+        bool h1 = box_hit(N, 1, f, tmin, limit, t1);
         if ((h0 && N.leaf(0)) || (h1 && N.leaf(1))) {
             int i, end;
             N.leaves(h0 && N.leaf(0), h1, i, end);
             for (; i < end && !hit; i += 2) {
-                const DrTri T0 = gptr(S.tris)[i], T1 = gptr(S.tris)[min(i + 1, end - 1)];
+                const DrTri T0 = gptr(S.tris)[i], T1 = gptr(S.tris)[i + 1];
                 float u, v, t;
-                nt += i + 1 < end ? 2 : 1;
-                const bool hit0 = tri_hit(T0, org, dir, tmin, tmax, u, v, t);
-                const bool hit1 = tri_hit(T1, org, dir, tmin, tmax, u, v, t);
-                hit = hit0 || hit1;
+                nt++;
+                hit = tri_hit(T0, org, dir, tmin, tmax, u, v, t);
+                if (!hit && i + 1 < end) {
+                    nt++;
+                    hit = tri_hit(T1, org, dir, tmin, tmax, u, v, t);
+                }
             }
             h0 = h0 && !N.leaf(0);
             h1 = false;

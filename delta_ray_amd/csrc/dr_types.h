@@ -40,15 +40,17 @@ struct DrNode {
 // What ray walks read of a node: the planes of both child boxes in bytes, on a
 // frame of the node's own (dr_bvh_pack.h), so that a box is wider than the
 // exact one by at most about a hundredth of its parent's at any scale of the
-// scene; half the bytes of a DrNode.  w[0..2]: the frame's origin; w[3]: its
-// steps (the top 9 bits of a float below its sign: x in bits 22-30, y 13-21, z
-// 4-12), bits 0-1 / 2-3: triangles of leaf 0 / 1 (0: not a leaf), bit 31: child 1
-// is a leaf; w[4..6]: per axis lo and hi of child 0, then of child 1; w[7]: the
-// first triangle slot of the leaves, or child 1's node.  Child 0's node is the
-// next one.
+// scene; half the bytes of a DrNode.  w[0..2]: the frame's origin, its lowest bit
+// the sign of the step; w[3]: the steps (the top 9 bits of a float below its sign: x
+// in bits 22-30, y 13-21, z 4-12), bits 0-1 / 2-3: triangles of leaf 0 / 1 (0: not a
+// leaf), bit 31: child 1 is a leaf; w[4..6]: per axis the near and far plane of child
+// 0, then of child 1; w[7]: the first triangle slot of the leaves, or child 1's node.
+// Child 0's node is the next one.
 struct alignas(16) DrPackedNode {
     uint32_t w[8];
 };
+// far planes lie this part of a step beyond origin + q * step
+#define DR_PACK_FAR 0.0009765625f
 
 struct DrTri {
     float v0[4];  // w: global triangle id (int bits)

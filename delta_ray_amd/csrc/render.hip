@@ -1727,7 +1727,10 @@ static bool upload_structures(dr_scene *s) {
     free_struct(s->st);
     SceneStruct &st = s->st;
     std::vector<void *> &A = st.allocs;
-    bool ok = upload_to(A, hs.nodes, &v.nodes) && upload_to(A, hs.tris, &v.tris) &&
+    // (ray walks load triangles in pairs: one more than there are)
+    std::vector<DrTri> tris(hs.tris);
+    if (!tris.empty()) tris.push_back(tris.back());
+    bool ok = upload_to(A, hs.nodes, &v.nodes) && upload_to(A, tris, &v.tris) &&
               upload_to(A, hs.sil_edges, &v.sil_edges) && upload_to(A, hs.sil_nodes, &v.sil_nodes) &&
               upload_to(A, hs.nrm_edges, &v.nrm_edges) && upload_to(A, hs.nrm_nodes, &v.nrm_nodes) &&
               upload_to(A, hs.nrm_geo, &v.nrm_geo) && upload_to(A, hs.sil_geo, &v.sil_geo) &&
