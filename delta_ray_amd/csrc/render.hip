@@ -208,7 +208,7 @@ DR_INLINE SelEntry sel_entry(int slot, const TreeEntry &e, TreeAlt a) {
 DR_INLINE TreeEntry sel_tree(const SelEntry &x) { return TreeEntry{x.code, x.cpmf, x.apmf, x.off}; }
 
 // the point's traversal state rebuilt from its SelPoint (what et_expand and
-// et_leaf read: tree, bound constants, light cone, proposal, keyed draws;
+// et_leaf_edge read: tree, bound constants, light cone, proposal, keyed draws;
 // of the surface point only its position and normal)
 DR_INLINE void sel_ctx(const SelPoint &P, const DrJob &J, EdgeTraversal &T, SPoint &sp) {
     const DrSceneView &S = J.S;

@@ -68,7 +68,7 @@ def test_batch_matches_single_renders(gpu):
 def test_batch_small_passes_match(gpu, refill):
     """Jobs split over many passes (tiny pass budget) give the same result,
     whatever the edge selection: breadth first (refill 0) or depth first
-    with 1 or 64 idle lanes gathered before new shading points start (the
+    with waves that take at most 1 or 64 shading points at a time (the
     schedule changes, the selected edges and the estimate do not)."""
     import torch
     jobs = _job_list(torch, gpu)
